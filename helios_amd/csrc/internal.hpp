@@ -247,13 +247,14 @@ struct Net {
     __bf16* xin = nullptr;
     float* resid = nullptr;   // float4 per pixel: log1p radiance
     float* out = nullptr;     // float4 per pixel: network output (log1p space)
-    float* dout = nullptr;
     __bf16* act[kDnLayers] = {nullptr};
     __bf16* pool[3] = {nullptr};
     __bf16* gy[2] = {nullptr, nullptr};
     float* gskip[3] = {nullptr};
     float* gpool[3] = {nullptr};
     float* loss = nullptr;
+    float* gpart = nullptr;   // partial gradients of one backward pass (workgroup slices)
+    size_t gpart_cap = 0;
 
     hipError_t init();
     hipError_t zero_state(hipStream_t st);

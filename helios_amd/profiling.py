@@ -135,7 +135,7 @@ def mfma_md(stats_csv, pmc_csv, cmd, peak_tflops=2500.0, simds=1024):
         # GRBM_GUI_ACTIVE is summed over the 8 XCDs
         util = 100.0 * busy / (gui / 8 * simds) if gui else 0.0
         lines.append(f"| {k} | {calls} | {ns / 1e3:.1f} | {flop / 1e9:.2f} | {flop / ns / 1e3:.1f} | {util:.1f} |")
-        if k not in ("hh::dn::k_relayout", "hh::dn::k_zero_f32", "hh::dn::k_to_bf16"):
+        if k not in ("hh::dn::k_relayout", "hh::dn::k_zero_f32"):
             tot_ns += ns * calls
             tot_flop += flop * calls
     lines += ["", f"Forward passes: {tot_flop / 1e9:.1f} GFLOP of MFMA work in {tot_ns / 1e6:.3f} ms of kernel time "

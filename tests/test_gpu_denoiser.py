@@ -113,6 +113,37 @@ def test_gradients_match_oracle(dn, kind):
             assert rel(a, b) <= 3e-2 and cos >= 0.999, (name, what, rel(a, b), cos)
 
 
+@pytest.mark.parametrize("n,h,w", [(1, 8, 16), (2, 24, 72), (1, 13, 21), (3, 40, 40), (140, 8, 8)])
+def test_gradients_at_strip_edges(dn, n, h, w):
+    """The weight gradient walks 32-pixel-wide strips: images narrower than a
+    strip (one pixel at the coarsest level), ragged last strips, padded sizes,
+    and more strips than workgroups. Bars as above: the sums themselves are
+    FP32, so only BF16 roundings of activations and their gradients differ."""
+    rng = np.random.default_rng(100 * n + h + w)
+    params = perturbed_params(7)
+    dn.set_params(unet.flatten(params).astype(np.float32))
+    feats = random_feats(rng, n, h, w)
+    target = rng.gamma(1.0, 0.4, size=(n, h, w, 3)).astype(np.float32)
+    loss = dn.loss_grad(feats, target)
+    g = unet.unflatten(dn.grads())
+    hp, wp = (h + 7) // 8 * 8, (w + 7) // 8 * 8
+    padded = np.zeros((n, hp, wp, unet.N_FEAT), np.float32)
+    padded[:, :h, :w] = feats
+    x = unet.pack_inputs(padded)
+    x[:, h:], x[:, :, w:] = 0.0, 0.0
+    out, cache = unet.forward(params, x, emulate_bf16=True)
+    ref_loss, d = unet.loss_mse(out[:, :h, :w], np.log1p(target.astype(np.float64)))
+    dout = np.zeros_like(out)
+    dout[:, :h, :w] = d
+    assert abs(loss - ref_loss) <= 1e-3 * ref_loss
+    ref = unet.backward(params, cache, dout)
+    for name, _, _ in unet.param_shapes():
+        for k, what in ((0, "W"), (1, "b")):
+            a, b = g[name][k], ref[name][k]
+            cos = float(np.dot(a.ravel(), b.ravel()) / (np.linalg.norm(a) * np.linalg.norm(b) + 1e-30))
+            assert rel(a, b) <= 3e-2 and cos >= 0.999, (name, what, rel(a, b), cos)
+
+
 def test_training_lowers_loss(gpu_ctx):
     """A fixed batch of noisy constant patches: 60 Adam steps cut the loss."""
     from helios_amd.denoise import Denoiser
