@@ -2360,7 +2360,7 @@ hipError_t hh::Wavefront::ensure(uint32_t n, uint64_t queue_entries) {
     HH_TRY(hipMalloc(&s_c, Q * 16));
     HH_TRY(hipMalloc(&s_slot, Q * 4));
     HH_TRY(hipMalloc(&feat, N * 32));
-    HH_TRY(hipMalloc(&counters, (size_t)kCtrKinds * kQShards * kCtrStride * 4));
+    HH_TRY(hipMalloc(&counters, kCtrWords * 4));
     HH_TRY(hipMalloc(&stats, 64));
     capacity = (uint32_t)N;
     qcap = Q;

@@ -71,8 +71,15 @@ hipError_t quantize_bvh4(hipStream_t st, const void* d_src, void* d_dst, uint32_
 // would serialize the per-wave allocations and refills of a whole frame.
 constexpr uint32_t kQShards = 32;
 constexpr uint32_t kCtrStride = 64;  // u32 words between two counters
-enum CtrKind : uint32_t { kCtrExt0 = 0, kCtrExt1 = 1, kCtrShadow = 2, kCtrExtHead = 3, kCtrShadowHead = 4, kCtrKinds = 5 };
-__host__ __device__ inline uint32_t ctr_index(uint32_t kind, uint32_t shard) { return (kind * kQShards + shard) * kCtrStride; }
+// Every bounce has counters of its own (lengths and read heads of its extension
+// and shadow queue), cleared together when a frame starts, so no launch between
+// two bounces has to reset any.
+enum CtrKind : uint32_t { kCtrExt = 0, kCtrExtHead = 1, kCtrShadow = 2, kCtrShadowHead = 3, kCtrKinds = 4 };
+constexpr uint32_t kMaxBounces = 64;
+constexpr size_t kCtrWords = (size_t)(kMaxBounces + 1) * kCtrKinds * kQShards * kCtrStride;
+__host__ __device__ inline uint32_t ctr_index(uint32_t depth, uint32_t kind, uint32_t shard) {
+    return ((depth * kCtrKinds + kind) * kQShards + shard) * kCtrStride;
+}
 
 // Entries per queue segment for `total` paths traced by a persistent grid of
 // `grid` blocks of `bs` threads. A producer wave w writes to segment w % kQShards
@@ -121,7 +128,7 @@ struct Wavefront {
     // first-hit features by slot, written at depth 0 when a view has feature
     // planes: feat[slot] = (albedo, 1/(1+t)), feat[capacity + slot] = (normal, 0)
     float4* feat = nullptr;
-    // kCtrKinds x kQShards counters, see ctr_index
+    // kCtrWords queue counters, see ctr_index
     uint32_t* counters = nullptr;
     unsigned long long* stats = nullptr;  // [0] extension rays, [1] shadow rays
     // traversal stack overflow, kSpillStackDepth words per launched thread

@@ -277,7 +277,7 @@ struct Tracer {
     // instance records, read once per instance entry, are reached through S)
     const HH_GLOBAL void* nodes;
     const HH_GLOBAL float4* tris;
-    f3 wo, wd, winv;   // world-space ray
+    f3 wo, wd;         // world-space ray
     f3 o, inv;         // ray in the current (world or instance) space
     WT wt;
     float tmin;
@@ -295,9 +295,8 @@ struct Tracer {
         tris = (const HH_GLOBAL float4*)scene.tris;
         wo = ro;
         wd = rd;
-        winv = box_inv(rd);
         o = wo;
-        inv = winv;
+        inv = box_inv(rd);
         wt = wt_pre(rd);
         tmin = t0;
         inst = -1;
@@ -500,7 +499,7 @@ struct Tracer {
         trips++;
         if (cur == kMarker) {
             o = wo;
-            inv = winv;
+            inv = box_inv(wd);   // three v_rcp_f32 again rather than three registers
             inst = -1;
             pop(stk);
         } else if (inst < 0) {
@@ -534,6 +533,256 @@ __device__ inline bool trace_ray(const SceneGPU& S, f3 wo, f3 wd, float tmin, fl
     h = tr.h;
     return h.found;
 }
+
+// ---------------------------------------------------------------------------
+// Four lanes per ray (BVH4), for launches with too few rays to fill the chip
+// with one lane each: lane k of a quad tests child k of the quad's node and
+// triangle k of its leaf, so a node visit is one box test instead of four and
+// a sort of four keys becomes three quad_perm comparisons, and a wave's lanes
+// diverge over 16 rays instead of 64. What bounds such launches is the serial
+// chain of one wave per SIMD (about eight cycles per instruction, no other
+// wave to hide a load behind), so fewer instructions per visit and four times
+// the waves shorten it. Full launches stay with one lane per ray: the
+// per-ray state and stack work of a quad is done four times over.
+//
+// Every lane of a quad holds the ray and the walk's state (so branches on
+// them are quad-uniform); each keeps the closest of the triangles it tested,
+// `tq` the closest distance of the quad. The result is the smallest (t,
+// instance, geometry, primitive) of the four, i.e. Tracer's.
+// ---------------------------------------------------------------------------
+constexpr int kQuadRays = 16;                                // rays per wave
+constexpr int kQuadLds = kLdsStack * 64 / kQuadRays;         // stack entries per ray in the wave's LDS
+constexpr int kQuadStack = kLdsStack + kSpillStack;          // capacity, as a lane's stack
+
+// Lane (l ^ 1), (l ^ 2), (l ^ 3) of the quad.
+template <int X>
+__device__ inline uint32_t quad_xor(uint32_t v) {
+    constexpr int ctrl = X == 1 ? 0xB1 : (X == 2 ? 0x4E : 0x1B);
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
+}
+template <int X>
+__device__ inline float quad_xor(float v) {
+    return __uint_as_float(quad_xor<X>(__float_as_uint(v)));
+}
+__device__ inline uint32_t quad_or(uint32_t v) {
+    v |= quad_xor<1>(v);
+    return v | quad_xor<2>(v);
+}
+
+// A quad's stack: entry e < kQuadLds at lds[e * 16] of the wave's area (the 16
+// quads of a wave interleaved, so their accesses fall on distinct banks),
+// deeper ones in a column of the launch's spill area of its own.
+struct QuadStack {
+    HH_LDS uint32_t* lds;
+    HH_GLOBAL uint32_t* spill;
+    uint32_t spill_stride;
+};
+// `stack` is the block's array of kLdsStack words per thread, `spill` the
+// launch's spill area (at most kQuadStack - kQuadLds words per ray).
+__device__ inline QuadStack quad_stack(uint32_t* stack, uint32_t* spill, uint32_t threads_per_block, uint32_t blocks) {
+    static_assert(kQuadStack - kQuadLds <= 4 * kSpillStack, "a quad's spill column fits its four lanes' share");
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    return {to_lds(stack + (t - lane) * kLdsStack + (lane >> 2)),
+            to_global(spill + ((blockIdx.x * threads_per_block + t) >> 2)), (threads_per_block * blocks) >> 2};
+}
+
+template <bool ANY>
+struct QuadTracer {
+    const SceneGPU* S;
+    const HH_GLOBAL void* nodes;
+    const HH_GLOBAL float4* tris;
+    f3 wo, wd;
+    f3 o, inv;
+    WT wt;
+    float tmin, tq;
+    int inst;
+    uint32_t sp, cur, trips;
+    bool alpha_on;
+    HitRec h;          // the closest of the triangles this lane tested; the quad's after finish()
+    uint32_t hgeom, hprim;
+
+    __device__ inline void begin(const SceneGPU& scene, f3 ro, f3 rd, float t0, float t1, uint32_t rflags) {
+        S = &scene;
+        nodes = (const HH_GLOBAL void*)scene.nodes;
+        tris = (const HH_GLOBAL float4*)scene.tris;
+        wo = ro;
+        wd = rd;
+        o = wo;
+        inv = box_inv(rd);
+        wt = wt_pre(rd);
+        tmin = t0;
+        tq = t1;
+        inst = -1;
+        sp = 0;
+        trips = 0;
+        alpha_on = (rflags & 1u) == 0u;
+        h.found = false;
+        h.t = t1;
+        h.u = h.v = 0.0f;
+        h.inst = 0xFFFFFFFFu;
+        h.tri = 0xFFFFFFFFu;
+        hgeom = hprim = 0xFFFFFFFFu;
+        cur = scene.tlas_root;
+    }
+    __device__ inline void store(const QuadStack& stk, uint32_t e, uint32_t r) {
+        if (e < (uint32_t)kQuadLds) stk.lds[e * kQuadRays] = r;
+        else if (e < (uint32_t)kQuadStack) stk.spill[(e - kQuadLds) * stk.spill_stride] = r;
+    }
+    __device__ inline uint32_t load(const QuadStack& stk, uint32_t e) {
+        uint32_t r = stk.lds[min(e, (uint32_t)kQuadLds - 1u) * kQuadRays];
+        if (e >= (uint32_t)kQuadLds) r = stk.spill[(e - kQuadLds) * stk.spill_stride];
+        return r;
+    }
+    __device__ inline void check_full() {
+        if (sp > (uint32_t)kQuadStack) {
+            trips = kStackFull;
+            sp = kQuadStack;
+        }
+    }
+    // What one lane stored, the others of its quad read: LDS and global
+    // accesses of a wave complete in order, the fence keeps the compiler's.
+    __device__ static inline void fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+    __device__ inline void pop(const QuadStack& stk) {
+        fence();
+        const uint32_t s = sp == 0u ? 0u : sp - 1u;
+        const uint32_t r = load(stk, s);
+        cur = sp == 0u ? kDone : r;
+        sp = s;
+    }
+
+    __device__ inline void visit_inner(const QuadStack& stk) {
+        fence();
+        const uint32_t k = __lane_id() & 3u;
+        const HH_GLOBAL float* p = (const HH_GLOBAL float*)nodes + 32 * (size_t)cur + k;
+        const float lox = p[0], hix = p[4], loy = p[8], hiy = p[12], loz = p[16], hiz = p[20];
+        const uint32_t ref = __float_as_uint(p[24]);
+        // the entry a pop would take, read while the node arrives
+        const uint32_t below = sp == 0u ? 0u : sp - 1u;
+        const uint32_t top = load(stk, below);
+        const float t = slab(lox, hix, loy, hiy, loz, hiz, o, inv, tmin, tq);
+        const bool hit = t != INFINITY;
+        // order within the quad: by entry distance (by child for any-hit
+        // rays), the child index breaking ties; misses last
+        const uint32_t key = hit ? (ANY ? k : ((__float_as_uint(t) & ~3u) | k)) : 0xFFFFFFFFu;
+        const uint32_t rank = (quad_xor<1>(key) < key ? 1u : 0u) + (quad_xor<2>(key) < key ? 1u : 0u) +
+                              (quad_xor<3>(key) < key ? 1u : 0u);
+        uint32_t nhit = hit ? 1u : 0u;
+        nhit += quad_xor<1>(nhit);
+        nhit += quad_xor<2>(nhit);
+        // the first child is visited next, the others pushed, the last deepest
+        if (hit && rank != 0u) store(stk, sp + nhit - 1u - rank, ref);
+        const uint32_t next = quad_or(hit && rank == 0u ? ref : 0u);
+        cur = nhit != 0u ? next : (sp == 0u ? kDone : top);
+        sp = nhit != 0u ? sp + nhit - 1u : below;
+        check_full();
+    }
+
+    // Triangles of leaf `cur`, four at a time; returns true when an any-hit
+    // ray found its occluder.
+    __device__ inline bool visit_leaf() {
+        const uint32_t first = leaf_start(cur), ntri = leaf_count(cur);
+        for (uint32_t k = __lane_id() & 3u; k < ntri; k += 4u) {
+            const uint32_t ti = first + k;
+            const float4 a = tris[3 * ti], b = tris[3 * ti + 1], c = tris[3 * ti + 2];
+            float t, u, v;
+            if (!tri_hit(wt, o, ld3(a), ld3(b), ld3(c), tmin, tq, t, u, v)) continue;
+            const uint32_t prim = __float_as_uint(a.w);
+            const uint32_t gw = __float_as_uint(b.w);
+            const uint32_t geom = gw & 0x7FFFFFFFu;
+            if (!ANY && h.found && (t > h.t || (t == h.t && !key_less((uint32_t)inst, geom, prim, h.inst, hgeom, hprim)))) continue;
+            if (alpha_on && (gw & 0x80000000u) == 0u) {
+                if (hit_alpha(*S, (uint32_t)inst, geom, ti, u, v) < 0.1f) continue;
+            }
+            h.found = true;
+            if (ANY) break;
+            h.t = t;
+            h.u = u;
+            h.v = v;
+            h.inst = (uint32_t)inst;
+            h.tri = ti;
+            hgeom = geom;
+            hprim = prim;
+        }
+        if (ANY) return quad_or(h.found ? 1u : 0u) != 0u;
+        tq = fminf(tq, h.t);
+        tq = fminf(tq, quad_xor<1>(tq));
+        tq = fminf(tq, quad_xor<2>(tq));
+        return false;
+    }
+
+    __device__ inline bool at_inner() const { return (int32_t)(cur | (trips << 9)) >= 0; }
+
+    // As Tracer::step<kWhileWhile>, a quad advancing together; returns true
+    // (in all four lanes) once the ray is finished.
+    __device__ inline bool step(const QuadStack& stk) {
+        unsigned long long mi = __builtin_amdgcn_ballot_w64(at_inner());
+        unsigned long long ml = __builtin_amdgcn_ballot_w64(cur != kDone);
+        while (mi != 0ull && (uint32_t)__popcll(ml) < (kLeafWait + 1u) * (uint32_t)__popcll(mi)) {
+            if (__builtin_amdgcn_inverse_ballot_w64(mi)) {
+                trips++;
+                visit_inner(stk);
+            }
+            mi = __builtin_amdgcn_ballot_w64(at_inner());
+            ml = __builtin_amdgcn_ballot_w64(cur != kDone);
+        }
+        if (at_inner()) return false;
+        if (cur == kDone) return true;
+        if (trips >= kMaxTrips) {
+            if ((__lane_id() & 3u) == 0u) atomicAdd(&S->faults[trips == kStackFull ? kFaultLaneStack : kFaultTrips], 1ull);
+            return true;
+        }
+        trips++;
+        if (cur == kMarker) {
+            o = wo;
+            inv = box_inv(wd);
+            inst = -1;
+            pop(stk);
+        } else if (inst < 0) {
+            inst = (int)leaf_start(cur);
+            const HH_GLOBAL InstTrav& it = ((const HH_GLOBAL InstTrav*)S->inst_trav)[inst];
+            f3 od;
+            xform_ray(it.w2o, wo, wd, o, od);
+            inv = box_inv(od);
+            wt = wt_pre(od);
+            if ((__lane_id() & 3u) == 0u) store(stk, sp, kMarker);
+            sp++;
+            check_full();
+            cur = it.blas_root;
+            return false;
+        } else {
+            if (visit_leaf()) return true;
+            pop(stk);
+        }
+        return cur == kDone;
+    }
+
+    // The quad's hit in all four lanes: the smallest (t, instance, geometry,
+    // primitive). For any-hit rays only h.found counts.
+    __device__ inline void finish() {
+        if (ANY) {
+            h.found = quad_or(h.found ? 1u : 0u) != 0u;
+            return;
+        }
+        take_better<1>();
+        take_better<2>();
+    }
+    template <int X>
+    __device__ inline void take_better() {
+        const uint32_t of = quad_xor<X>(h.found ? 1u : 0u), oi = quad_xor<X>(h.inst), ot = quad_xor<X>(h.tri),
+                       og = quad_xor<X>(hgeom), op = quad_xor<X>(hprim);
+        const float t = quad_xor<X>(h.t), u = quad_xor<X>(h.u), v = quad_xor<X>(h.v);
+        if (of != 0u && (!h.found || t < h.t || (t == h.t && key_less(oi, og, op, h.inst, hgeom, hprim)))) {
+            h.found = true;
+            h.t = t;
+            h.u = u;
+            h.v = v;
+            h.inst = oi;
+            h.tri = ot;
+            hgeom = og;
+            hprim = op;
+        }
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Packet traversal for neighbouring camera rays (the 64 lanes of a wave hold
