@@ -20,7 +20,6 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/helios_hip.h"
@@ -936,79 +935,65 @@ hh_status hh_scene_commit(hh_scene s) {
     // positions): (u0 v0 u1 v1) (u2 v2 n0.x n0.y) (n0.z n1.xyz) (n2.xyz 0), the
     // vertex attributes the shading and the alpha test interpolate, in one
     // line. Mesh g owns triangles tri_off[g]..; an empty mesh one inert
-    // triangle. Filled by host threads, one mesh at a time per thread.
+    // triangle. Gathered on the GPU from the vertex and index pools; the host
+    // builder's copy of the positions is filled on the host.
     const size_t G = global_meshes.size();
     std::vector<uint32_t> tri_off(G + 1, 0);
     for (size_t g = 0; g < G; g++) tri_off[g + 1] = tri_off[g] + mesh_tris[g];
-    std::vector<float4> soup(ntri * 3), shade_soup(ntri * 4);
-    auto fill_mesh = [&](size_t g) {
+    auto geom_word = [&](const MeshHost& me, uint32_t gi) -> uint32_t {
+        const hh_material_desc& m = s->materials[me.mats[me.sm[gi].mat_idx]];
+        return gi | ((m.type == HH_MATERIAL_OPAQUE && !m.alpha_test) ? 0x80000000u : 0u);  // mesh.cpp:75-76
+    };
+    std::vector<SoupRange> soup_ranges;
+    for (size_t g = 0; g < G; g++) {
         const MeshHost& me = s->meshes[global_meshes[g]];
-        float4* ps = &soup[3 * size_t(tri_off[g])];
-        float4* ss = &shade_soup[4 * size_t(tri_off[g])];
-        size_t t = 0;
+        uint32_t t = tri_off[g];
         for (uint32_t gi = 0; gi < me.sm.size(); gi++) {
             const hh_submesh& sm = me.sm[gi];
-            const hh_material_desc& m = s->materials[me.mats[sm.mat_idx]];
-            uint32_t opaque = (m.type == HH_MATERIAL_OPAQUE && !m.alpha_test) ? 0x80000000u : 0u;  // mesh.cpp:75-76
-            for (uint32_t p = 0; p < sm.index_count / 3; p++, t++) {
-                const hh_vertex* v3[3];
-                for (int k = 0; k < 3; k++) v3[k] = &me.v[me.idx[sm.base_index + 3 * p + k]];
-                uint32_t w0 = p, w1 = gi | opaque;
-                float fw0, fw1;
-                std::memcpy(&fw0, &w0, 4);
-                std::memcpy(&fw1, &w1, 4);
-                ps[3 * t] = make_float4(v3[0]->position[0], v3[0]->position[1], v3[0]->position[2], fw0);
-                ps[3 * t + 1] = make_float4(v3[1]->position[0], v3[1]->position[1], v3[1]->position[2], fw1);
-                ps[3 * t + 2] = make_float4(v3[2]->position[0], v3[2]->position[1], v3[2]->position[2], 0.f);
-                ss[4 * t] = make_float4(v3[0]->tex_coord[0], v3[0]->tex_coord[1], v3[1]->tex_coord[0], v3[1]->tex_coord[1]);
-                ss[4 * t + 1] = make_float4(v3[2]->tex_coord[0], v3[2]->tex_coord[1], v3[0]->normal[0], v3[0]->normal[1]);
-                ss[4 * t + 2] = make_float4(v3[0]->normal[2], v3[1]->normal[0], v3[1]->normal[1], v3[1]->normal[2]);
-                ss[4 * t + 3] = make_float4(v3[2]->normal[0], v3[2]->normal[1], v3[2]->normal[2], 0.f);
-            }
+            if (sm.index_count == 0) continue;
+            soup_ranges.push_back({t, ibase[g] + sm.base_index, vbase[g], geom_word(me, gi)});
+            t += sm.index_count / 3;
         }
-        if (t == 0) {
-            for (int k = 0; k < 3; k++) ps[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-            for (int k = 0; k < 4; k++) ss[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (t == tri_off[g]) soup_ranges.push_back({t, kInertSoup, 0u, 0u});
+    }
+    std::vector<float4> soup;
+    if (ctx->tune.bvh_builder == 1) {   // the host builder reads the triangles
+        soup.assign(ntri * 3, make_float4(0.f, 0.f, 0.f, 0.f));
+        for (size_t g = 0; g < G; g++) {
+            const MeshHost& me = s->meshes[global_meshes[g]];
+            float4* ps = &soup[3 * size_t(tri_off[g])];
+            for (const hh_submesh& sm : me.sm)
+                for (uint32_t k = 0; k < sm.index_count; k++, ps++) {
+                    const float* p = me.v[me.idx[sm.base_index + k]].position;
+                    *ps = make_float4(p[0], p[1], p[2], 0.f);
+                }
         }
-    };
-    {
-        const size_t nth = std::min<size_t>(G, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
-        std::vector<std::thread> pool;
-        for (size_t w = 1; w < nth; w++)
-            pool.emplace_back([&, w] {
-                for (size_t g = w; g < G; g += nth) fill_mesh(g);
-            });
-        for (size_t g = 0; g < G; g += nth) fill_mesh(g);
-        for (auto& th : pool) th.join();
     }
     float4* d_soup = nullptr;
     float4* d_shade_soup = nullptr;
-    HH_HIP(hipMalloc(&d_soup, soup.size() * sizeof(float4)));
-    if (hipMalloc(&d_shade_soup, shade_soup.size() * sizeof(float4)) != hipSuccess) {
-        (void)hipFree(d_soup);
-        return fail(HH_ERR_OUT_OF_MEMORY, "shading records");
-    }
-    hipError_t e = hipSuccess;
-    if (ntri > 0) {
-        e = hipMemcpyAsync(d_soup, soup.data(), soup.size() * sizeof(float4), hipMemcpyHostToDevice, ctx->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(d_shade_soup, shade_soup.data(), shade_soup.size() * sizeof(float4), hipMemcpyHostToDevice,
-                               ctx->stream);
-    }
+    SoupRange* d_ranges = nullptr;
+    hipError_t e = hipMalloc(&d_soup, std::max<size_t>(ntri, 1) * 3 * sizeof(float4));
+    if (e == hipSuccess) e = hipMalloc(&d_shade_soup, std::max<size_t>(ntri, 1) * 4 * sizeof(float4));
+    if (e == hipSuccess) e = hipMalloc(&d_ranges, std::max<size_t>(soup_ranges.size(), 1) * sizeof(SoupRange));
+    if (e == hipSuccess && !soup_ranges.empty())
+        e = hipMemcpyAsync(d_ranges, soup_ranges.data(), soup_ranges.size() * sizeof(SoupRange), hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess)
+        e = launch_soup(ctx->stream, d_ranges, (uint32_t)soup_ranges.size(), (uint32_t)ntri, d_vtx, d_idx, d_soup, d_shade_soup);
     hh_status st = HH_OK;
     if (e != hipSuccess) {
-        st = hip_fail(e, "triangle upload");
+        st = hip_fail(e, "triangle records");
     } else if (G == 0) {
         // no meshes: no BLAS
     } else if (ctx->tune.bvh_builder == 3) {
         // every mesh's tree on the GPU together
         std::vector<int2> ranges(G);
-        std::vector<uint32_t> counts(G);
-        for (size_t g = 0; g < G; g++) ranges[g] = make_int2((int)tri_off[g], (int)mesh_tris[g]);
+        for (size_t g = 0; g < G; g++) {
+            ranges[g] = make_int2((int)tri_off[g], (int)mesh_tris[g]);
+            blas_root[g] = (uint32_t)g;
+        }
         e = build_blas_forest(ctx->stream, W, ctx->tune.leaf_size, ranges, (uint32_t)ntri, d_soup, d_tris, d_shade_soup,
-                              d_shade, d_nodes, 0, ctx->bs, blas_root.data(), counts.data(), blas_box.data());
+                              d_shade, d_nodes, 0, ctx->bs, &node_base, blas_box.data());
         if (e != hipSuccess) st = hip_fail(e, "BLAS build");
-        for (uint32_t c : counts) node_base += c;
         tri_base = (uint32_t)ntri;
     } else {
         for (size_t g = 0; g < G; g++) {
@@ -1028,8 +1013,9 @@ hh_status hh_scene_commit(hh_scene s) {
         }
     }
     (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(d_soup);
-    (void)hipFree(d_shade_soup);
+    if (d_soup) (void)hipFree(d_soup);
+    if (d_shade_soup) (void)hipFree(d_shade_soup);
+    if (d_ranges) (void)hipFree(d_ranges);
     if (st != HH_OK) return st;
     s->bvh_stats[0] = node_base;
     s->bvh_stats[1] = tri_base;

@@ -171,13 +171,39 @@ __device__ inline float4 aload4(const float4* p) {
     return r;
 }
 
+// The last of nm ranges (first primitive, count) whose first element, scaled
+// by `scale`, is not above i.
+__device__ inline int2 range_of(const int2* __restrict__ ranges, int nm, int i, int scale) {
+    int lo = 0, hi = nm - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (scale * ranges[mid].x <= i) lo = mid;
+        else hi = mid - 1;
+    }
+    return ranges[lo];
+}
+
 // Bottom-up bounds: node boxes live in blo/bhi indexed by binary ref
 // (internal 0..n-2, leaves n-1..2n-2); .w of blo holds the primitive count.
+// With `ranges`, n primitives hold the trees of nm meshes: the tree of range
+// (P, m) has its leaves and internal nodes at P.. and its boxes and parents at
+// 2P.. of the arrays, numbered from 0 there.
 __global__ void k_refit(const float4* __restrict__ plo, const float4* __restrict__ phi, const uint32_t* __restrict__ order,
                         int n, const int2* __restrict__ childs, const uint32_t* __restrict__ parent, uint32_t* __restrict__ flags,
-                        float4* blo, float4* bhi) {
+                        float4* blo, float4* bhi, const int2* __restrict__ ranges, int nm) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
+    if (ranges) {
+        const int2 m = range_of(ranges, nm, j, 1);
+        j -= m.x;
+        n = m.y;
+        order += m.x;
+        childs += m.x;
+        flags += m.x;
+        parent += 2 * (size_t)m.x;
+        blo += 2 * (size_t)m.x;
+        bhi += 2 * (size_t)m.x;
+    }
     uint32_t p = order[j];
     float4 l = plo[p], h = phi[p];
     l.w = 1.0f;
@@ -215,17 +241,32 @@ __device__ inline float half_area(float4 l, float4 h) {
     return dx * dy + dy * dz + dz * dx;
 }
 
-// One wide node per job: job = (binary ref, wide index).
+// One wide node per job: job = (binary ref, wide index). With `ranges` (see
+// k_refit) a job's binary ref counts from the box array's start, which names
+// its mesh, and the leaves of a mesh start at its first primitive.
 template <int W>
 __global__ void k_collapse(const int2* __restrict__ jobs, const uint32_t* __restrict__ njobs_p, int2* __restrict__ out_jobs,
                            uint32_t* __restrict__ out_njobs, uint32_t* __restrict__ node_counter, int n, int leaf_size,
                            const int2* __restrict__ childs, const int2* __restrict__ range, const float4* __restrict__ blo,
                            const float4* __restrict__ bhi, const uint32_t* __restrict__ order, WideNode<W>* __restrict__ nodes,
-                           uint32_t node_base, uint32_t leaf_base, int leaf_is_prim) {
+                           uint32_t node_base, uint32_t leaf_base, int leaf_is_prim, const int2* __restrict__ ranges,
+                           int nm) {
     uint32_t jid = blockIdx.x * blockDim.x + threadIdx.x;
     if (jid >= *njobs_p) return;
     int2 job = jobs[jid];
-    int bref = job.x;
+    int bref = job.x, ref0 = 0;   // ref0: the mesh's first binary ref
+    if (ranges) {
+        const int2 m = range_of(ranges, nm, bref, 2);
+        ref0 = 2 * m.x;
+        bref -= ref0;
+        n = m.y;
+        childs += m.x;
+        range += m.x;
+        order += m.x;
+        blo += ref0;
+        bhi += ref0;
+        leaf_base = (uint32_t)m.x;
+    }
     auto is_internal = [&](int r) { return r < n - 1; };
     auto count_of = [&](int r) { return is_internal(r) ? (int)blo[r].w : 1; };
     auto expandable = [&](int r) { return is_internal(r) && count_of(r) > leaf_size; };
@@ -268,7 +309,7 @@ __global__ void k_collapse(const int2* __restrict__ jobs, const uint32_t* __rest
         if (expandable(r)) {
             uint32_t idx = atomicAdd(node_counter, 1u);
             uint32_t slot = atomicAdd(out_njobs, 1u);
-            out_jobs[slot] = make_int2(r, (int)idx);
+            out_jobs[slot] = make_int2(ref0 + r, (int)idx);
             nd.child[k] = node_base + idx;
         } else {
             int first, cnt;
@@ -278,6 +319,44 @@ __global__ void k_collapse(const int2* __restrict__ jobs, const uint32_t* __rest
         }
     }
     nodes[job.y] = nd;
+}
+
+// Triangles and shading records (gpu_scene.hpp) of every submesh from the
+// vertex and index pools, one thread per triangle.
+__global__ void k_soup(const SoupRange* __restrict__ ranges, int nr, uint32_t n, const float4* __restrict__ vtx,
+                       const uint32_t* __restrict__ idx, float4* __restrict__ tri, float4* __restrict__ shade) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    int lo = 0, hi = nr - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (ranges[mid].first <= i) lo = mid;
+        else hi = mid - 1;
+    }
+    const SoupRange r = ranges[lo];
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (r.index == kInertSoup) {
+        for (int k = 0; k < 3; k++) tri[3 * (size_t)i + k] = zero;
+        for (int k = 0; k < 4; k++) shade[4 * (size_t)i + k] = zero;
+        return;
+    }
+    const uint32_t p = i - r.first;
+    const uint32_t* ix = idx + (size_t)r.index + 3 * (size_t)p;
+    float4 pos[3], uv[3], nrm[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const float4* v = vtx + 5 * ((size_t)r.vertex + ix[k]);
+        pos[k] = v[0];
+        uv[k] = v[1];
+        nrm[k] = v[2];
+    }
+    tri[3 * (size_t)i] = make_float4(pos[0].x, pos[0].y, pos[0].z, __uint_as_float(p));
+    tri[3 * (size_t)i + 1] = make_float4(pos[1].x, pos[1].y, pos[1].z, __uint_as_float(r.geom));
+    tri[3 * (size_t)i + 2] = make_float4(pos[2].x, pos[2].y, pos[2].z, 0.f);
+    shade[4 * (size_t)i] = make_float4(uv[0].x, uv[0].y, uv[1].x, uv[1].y);
+    shade[4 * (size_t)i + 1] = make_float4(uv[2].x, uv[2].y, nrm[0].x, nrm[0].y);
+    shade[4 * (size_t)i + 2] = make_float4(nrm[0].z, nrm[1].x, nrm[1].y, nrm[1].z);
+    shade[4 * (size_t)i + 3] = make_float4(nrm[2].x, nrm[2].y, nrm[2].z, 0.f);
 }
 
 __global__ void k_gather_tris(const float4* __restrict__ src, const uint32_t* __restrict__ order, uint32_t n,
@@ -1142,6 +1221,31 @@ static hipError_t sah_forest_gpu(hipStream_t st, const std::vector<int2>& meshes
                                  const float4* d_hi, uint32_t* d_order, int2* childs, int2* range, uint32_t* parent,
                                  BuildScratch& sc);
 
+// The W-wide collapse, level by level, of the `njobs` roots in sc.jobs_a, which
+// take nodes 0..njobs-1; leaves the node count in sc.counters[2].
+template <int W>
+static hipError_t collapse_jobs(hipStream_t st, uint32_t njobs, uint32_t n, const uint32_t* d_order, const int2* childs,
+                                const int2* range, const float4* blo, const float4* bhi, BuildScratch& sc, int leaf_size,
+                                int leaf_is_prim, WideNode<W>* d_nodes, uint32_t node_base, uint32_t leaf_base,
+                                const int2* ranges, int nm) {
+    const uint32_t ctr[3] = {njobs, 0u, njobs};   // jobs in A, jobs in B, nodes
+    HH_TRY(hipMemcpyAsync(sc.counters, ctr, sizeof(ctr), hipMemcpyHostToDevice, st));
+    int2* qa = sc.jobs_a;
+    int2* qb = sc.jobs_b;
+    uint32_t* ca = sc.counters;
+    uint32_t* cb = sc.counters + 1;
+    while (njobs > 0) {
+        k_fill_u32<<<1, 1, 0, st>>>(cb, 0u, 1);
+        k_collapse<W><<<blocks(njobs, 64), 64, 0, st>>>(qa, ca, qb, cb, sc.counters + 2, (int)n, leaf_size, childs, range, blo,
+                                                         bhi, d_order, d_nodes, node_base, leaf_base, leaf_is_prim, ranges, nm);
+        HH_TRY(hipMemcpyAsync(&njobs, cb, 4, hipMemcpyDeviceToHost, st));
+        HH_TRY(hipStreamSynchronize(st));
+        std::swap(qa, qb);
+        std::swap(ca, cb);
+    }
+    return hipSuccess;
+}
+
 // Bounds (refit) and the W-wide collapse of one binary tree in the radix
 // tree's form over n primitives: `order` maps leaf positions to indices into
 // d_lo / d_hi; childs / range / flags hold n - 1 entries, parent / blo / bhi
@@ -1153,26 +1257,11 @@ static hipError_t finish_wide(hipStream_t st, uint32_t n, const float4* d_lo, co
                               float4* bhi, BuildScratch& sc, int leaf_size, int leaf_is_prim, WideNode<W>* d_nodes,
                               uint32_t node_base, uint32_t leaf_base, uint32_t* num_nodes, float root_box[6]) {
     const uint32_t B = 256;
-    k_refit<<<blocks(n, B), B, 0, st>>>(d_lo, d_hi, d_order, (int)n, childs, parent, flags, blo, bhi);
-    int2 job0 = make_int2(0, 0);   // binary ref of the root (leaf 0 when n == 1: ref n-1+0 = 0)
-    uint32_t one = 1;
+    k_refit<<<blocks(n, B), B, 0, st>>>(d_lo, d_hi, d_order, (int)n, childs, parent, flags, blo, bhi, nullptr, 0);
+    const int2 job0 = make_int2(0, 0);   // binary ref of the root (leaf 0 when n == 1: ref n-1+0 = 0)
     HH_TRY(hipMemcpyAsync(sc.jobs_a, &job0, sizeof(int2), hipMemcpyHostToDevice, st));
-    HH_TRY(hipMemcpyAsync(sc.counters, &one, 4, hipMemcpyHostToDevice, st));       // jobs in A
-    HH_TRY(hipMemcpyAsync(sc.counters + 2, &one, 4, hipMemcpyHostToDevice, st));   // node counter
-    uint32_t njobs = 1;
-    int2* qa = sc.jobs_a;
-    int2* qb = sc.jobs_b;
-    uint32_t* ca = sc.counters;
-    uint32_t* cb = sc.counters + 1;
-    while (njobs > 0) {
-        k_fill_u32<<<1, 1, 0, st>>>(cb, 0u, 1);
-        k_collapse<W><<<blocks(njobs, 64), 64, 0, st>>>(qa, ca, qb, cb, sc.counters + 2, (int)n, leaf_size, childs, range, blo,
-                                                         bhi, d_order, d_nodes, node_base, leaf_base, leaf_is_prim);
-        HH_TRY(hipMemcpyAsync(&njobs, cb, 4, hipMemcpyDeviceToHost, st));
-        HH_TRY(hipStreamSynchronize(st));
-        std::swap(qa, qb);
-        std::swap(ca, cb);
-    }
+    HH_TRY(collapse_jobs<W>(st, 1, n, d_order, childs, range, blo, bhi, sc, leaf_size, leaf_is_prim, d_nodes, node_base,
+                            leaf_base, nullptr, 0));
     HH_TRY(hipMemcpyAsync(num_nodes, sc.counters + 2, 4, hipMemcpyDeviceToHost, st));
     float4 rb[2];
     HH_TRY(hipMemcpyAsync(&rb[0], &blo[0], 16, hipMemcpyDeviceToHost, st));
@@ -1500,36 +1589,73 @@ hipError_t build_blas(hipStream_t st, int width, int leaf_size, uint32_t n, cons
 // per mesh the bounds and the wide collapse, whose nodes start at
 // node_base (advancing mesh by mesh: roots[g], counts[g]); then the
 // triangles and shading records of all meshes are gathered into leaf order.
+// The roots' boxes of a forest (see k_refit), two float4 per mesh.
+__global__ void k_root_boxes(const int2* __restrict__ ranges, int nm, const float4* __restrict__ blo,
+                             const float4* __restrict__ bhi, float4* __restrict__ out) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= nm) return;
+    out[2 * g] = blo[2 * (size_t)ranges[g].x];
+    out[2 * g + 1] = bhi[2 * (size_t)ranges[g].x];
+}
+
+template <int W>
+static hipError_t forest_wide(hipStream_t st, const std::vector<int2>& meshes, uint32_t total, BuildScratch& sc, int leaf_size,
+                              WideNode<W>* d_nodes, uint32_t node_base, uint32_t* num_nodes, float* root_boxes) {
+    const uint32_t B = 256, G = (uint32_t)meshes.size();
+    const int2* ranges = sc.s_meshes;
+    k_fill_u32<<<blocks(total, B), B, 0, st>>>(sc.flags, 0u, total);
+    k_refit<<<blocks(total, B), B, 0, st>>>(sc.aabb_lo, sc.aabb_hi, sc.order, (int)total, sc.childs, sc.parent, sc.flags, sc.blo,
+                                            sc.bhi, ranges, (int)G);
+    std::vector<int2> roots(G);
+    for (uint32_t g = 0; g < G; g++) roots[g] = make_int2(2 * meshes[g].x, (int)g);
+    HH_TRY(hipMemcpyAsync(sc.jobs_a, roots.data(), G * sizeof(int2), hipMemcpyHostToDevice, st));
+    HH_TRY(collapse_jobs<W>(st, G, total, sc.order, sc.childs, sc.range, sc.blo, sc.bhi, sc, leaf_size, 0, d_nodes, node_base, 0,
+                            ranges, (int)G));
+    k_root_boxes<<<blocks(G, 64), 64, 0, st>>>(ranges, (int)G, sc.blo, sc.bhi, sc.aabb_lo);
+    std::vector<float4> boxes(2 * (size_t)G);
+    HH_TRY(hipMemcpyAsync(num_nodes, sc.counters + 2, 4, hipMemcpyDeviceToHost, st));
+    HH_TRY(hipMemcpyAsync(boxes.data(), sc.aabb_lo, boxes.size() * sizeof(float4), hipMemcpyDeviceToHost, st));
+    HH_TRY(hipStreamSynchronize(st));
+    for (uint32_t g = 0; g < G; g++) {
+        const float4 l = boxes[2 * g], h = boxes[2 * g + 1];
+        const float b[6] = {l.x, l.y, l.z, h.x, h.y, h.z};
+        std::copy(b, b + 6, root_boxes + 6 * g);
+    }
+    return hipSuccess;
+}
+
+// Every mesh's binned-SAH tree in one build over the triangles of all of them
+// (meshes: first triangle and count, each count >= 1): splits, bounds and the
+// wide collapse go through each level of all trees together, so a build takes
+// about ten host round trips instead of ten per mesh. Mesh g's root is node
+// node_base + g. 50 meshes of 249 K triangles: COLLAPSEFIG
 hipError_t build_blas_forest(hipStream_t st, int width, int leaf_size, const std::vector<int2>& meshes, uint32_t total,
                              const float4* d_tri_src, float4* d_tri_pool, const float4* d_shade_src, float4* d_shade_pool,
-                             void* d_node_pool, uint32_t node_base, BuildScratch& sc, uint32_t* roots, uint32_t* counts,
+                             void* d_node_pool, uint32_t node_base, BuildScratch& sc, uint32_t* num_nodes,
                              float* root_boxes) {
+    *num_nodes = 0;
     if (meshes.empty() || total == 0) return hipSuccess;
-    HH_TRY(sc.ensure(total));
+    // k_root_boxes reuses the primitive boxes for two float4 per mesh
+    HH_TRY(sc.ensure(std::max<uint32_t>(total, 2 * (uint32_t)meshes.size())));
     const uint32_t B = 256;
     k_init_bounds<<<1, 64, 0, st>>>(sc.cbounds);
     k_tri_aabbs<<<blocks(total, B), B, 0, st>>>(d_tri_src, total, sc.aabb_lo, sc.aabb_hi, sc.cbounds);
     HH_TRY(sah_forest_gpu(st, meshes, total, sc.aabb_lo, sc.aabb_hi, sc.order, sc.childs, sc.range, sc.parent, sc));
-    k_fill_u32<<<blocks(total, B), B, 0, st>>>(sc.flags, 0u, total);
-    for (size_t g = 0; g < meshes.size(); g++) {
-        const uint32_t P = (uint32_t)meshes[g].x, n = (uint32_t)meshes[g].y;
-        uint32_t nn = 0;
-        hipError_t e;
-        if (width == 8)
-            e = finish_wide<8>(st, n, sc.aabb_lo, sc.aabb_hi, sc.order + P, sc.childs + P, sc.range + P, sc.parent + 2 * (size_t)P,
-                               sc.flags + P, sc.blo + 2 * (size_t)P, sc.bhi + 2 * (size_t)P, sc, leaf_size, 0,
-                               (WideNode<8>*)d_node_pool + node_base, node_base, P, &nn, root_boxes + 6 * g);
-        else
-            e = finish_wide<4>(st, n, sc.aabb_lo, sc.aabb_hi, sc.order + P, sc.childs + P, sc.range + P, sc.parent + 2 * (size_t)P,
-                               sc.flags + P, sc.blo + 2 * (size_t)P, sc.bhi + 2 * (size_t)P, sc, leaf_size, 0,
-                               (WideNode<4>*)d_node_pool + node_base, node_base, P, &nn, root_boxes + 6 * g);
-        HH_TRY(e);
-        roots[g] = node_base;
-        counts[g] = nn;
-        node_base += nn;
-    }
+    hipError_t e;
+    if (width == 8)
+        e = forest_wide<8>(st, meshes, total, sc, leaf_size, (WideNode<8>*)d_node_pool + node_base, node_base, num_nodes, root_boxes);
+    else
+        e = forest_wide<4>(st, meshes, total, sc, leaf_size, (WideNode<4>*)d_node_pool + node_base, node_base, num_nodes, root_boxes);
+    HH_TRY(e);
     k_gather_tris<<<blocks(total, B), B, 0, st>>>(d_tri_src, sc.order, total, d_tri_pool);
     k_gather_shade<<<blocks(total, B), B, 0, st>>>(d_shade_src, sc.order, total, d_shade_pool);
+    return hipGetLastError();
+}
+
+hipError_t launch_soup(hipStream_t st, const SoupRange* d_ranges, uint32_t nr, uint32_t n, const float4* d_vtx,
+                       const uint32_t* d_idx, float4* d_tri, float4* d_shade) {
+    if (n == 0 || nr == 0) return hipSuccess;
+    k_soup<<<(n + 255) / 256, 256, 0, st>>>(d_ranges, (int)nr, n, d_vtx, d_idx, d_tri, d_shade);
     return hipGetLastError();
 }
 

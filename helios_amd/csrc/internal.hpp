@@ -60,8 +60,16 @@ hipError_t build_tlas(hipStream_t st, int width, uint32_t n, const float* h_lo, 
                       uint32_t node_base, BuildScratch& sc, uint32_t* num_nodes, bool sah, bool ploc, bool sah_gpu);
 hipError_t build_blas_forest(hipStream_t st, int width, int leaf_size, const std::vector<int2>& meshes, uint32_t total,
                              const float4* d_tri_src, float4* d_tri_pool, const float4* d_shade_src, float4* d_shade_pool,
-                             void* d_node_pool, uint32_t node_base, BuildScratch& sc, uint32_t* roots, uint32_t* counts,
-                             float* root_boxes);
+                             void* d_node_pool, uint32_t node_base, BuildScratch& sc, uint32_t* num_nodes, float* root_boxes);
+// Triangles `first`.. of the soup are the triangles of one submesh: its first
+// index in the index pool, its mesh's first vertex, and its geometry word
+// (submesh | opaque bit). kInertSoup as index: one inert triangle.
+struct SoupRange {
+    uint32_t first, index, vertex, geom;
+};
+constexpr uint32_t kInertSoup = 0xFFFFFFFFu;
+hipError_t launch_soup(hipStream_t st, const SoupRange* d_ranges, uint32_t nr, uint32_t n, const float4* d_vtx,
+                       const uint32_t* d_idx, float4* d_tri, float4* d_shade);
 hipError_t quantize_bvh4(hipStream_t st, const void* d_src, void* d_dst, uint32_t n);
 
 // Ray queues are split into kQShards segments, each with its own length and
