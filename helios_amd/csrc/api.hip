@@ -62,6 +62,7 @@ static hh_status hip_fail(hipError_t e, const char* what) {
 // ---------------------------------------------------------------------------
 // Objects
 // ---------------------------------------------------------------------------
+constexpr size_t kMaxGraphs = 64;   // captured launch sequences a context keeps
 struct GraphEntry {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -143,18 +144,62 @@ struct hh_scene_t {
     uint64_t generation = 0;
     bool committed = false;
     bool dirty = true;
-    std::vector<void*> allocs;
+    // Device memory by what it is made from, so that a commit rebuilds only what
+    // its edits touch: the geometry (vertex, index, triangle and node pools,
+    // textures) after a mesh, material, texture or instance was added or the
+    // BVH tuning changed; the environment after a light, sky or IBL edit; the
+    // tables (instances, lights, materials, offsets) and the TLAS every time.
+    struct Geometry {
+        bool built = false;
+        int width = 0;
+        uint32_t builder = 0;
+        bool compressed = false;
+        std::vector<void*> allocs;
+        float4 *vtx = nullptr, *tris = nullptr, *shade = nullptr, *texels = nullptr;
+        uint32_t *idx = nullptr, *vbase = nullptr, *ibase = nullptr;
+        TexDesc* tex = nullptr;
+        void *nodes = nullptr, *qnodes = nullptr;
+        uint32_t num_nodes = 0, num_tris = 0;   // BLAS nodes, triangles
+        std::vector<uint32_t> blas_root;
+        std::vector<float> blas_box;
+    } geom;
+    struct Environment {
+        bool built = false;
+        std::vector<void*> allocs;
+        float4* cube = nullptr;
+        uint16_t* eq = nullptr;
+        uint32_t size = 0, eq_w = 0;
+    } env;
+    unsigned char* tables = nullptr;
+    size_t tables_cap = 0;
     SceneGPU gpu{};
     SceneGPU* d_gpu = nullptr;
     std::vector<LightData> light_data;
     float sky_coef[30] = {0};
     uint64_t bvh_stats[4] = {0, 0, 0, 0};
 
+    void free_geometry() {
+        for (void* p : geom.allocs) (void)hipFree(p);
+        geom = Geometry{};
+    }
+    void free_environment() {
+        for (void* p : env.allocs) (void)hipFree(p);
+        env = Environment{};
+    }
     void free_device() {
-        for (void* p : allocs) (void)hipFree(p);
-        allocs.clear();
+        free_geometry();
+        free_environment();
+        if (tables) (void)hipFree(tables);
+        tables = nullptr;
+        tables_cap = 0;
         d_gpu = nullptr;
         committed = false;
+    }
+    // An edit of the scene: what it needs rebuilt at the next commit.
+    void edited(bool geometry, bool environment) {
+        dirty = true;
+        if (geometry) geom.built = false;
+        if (environment) env.built = false;
     }
 };
 
@@ -325,21 +370,32 @@ bool material_is_emissive(const hh_material_desc& m) {  // material.cpp:71-77
 }  // namespace
 
 template <typename T>
-static hipError_t upload(hh_scene s, const std::vector<T>& v, T** out) {
-    size_t bytes = std::max<size_t>(v.size() * sizeof(T), 16);
+static hipError_t dalloc(std::vector<void*>& allocs, size_t count, T** out) {
     void* p = nullptr;
-    HH_TRY(hipMalloc(&p, bytes));
-    s->allocs.push_back(p);
-    if (!v.empty()) HH_TRY(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s->ctx->stream));
+    HH_TRY(hipMalloc(&p, std::max<size_t>(count * sizeof(T), 16)));
+    allocs.push_back(p);
     *out = (T*)p;
     return hipSuccess;
 }
-
-static hipError_t dalloc(hh_scene s, size_t bytes, void** out) {
-    HH_TRY(hipMalloc(out, std::max<size_t>(bytes, 16)));
-    s->allocs.push_back(*out);
+// A host array copied to a new allocation (the caller synchronizes before it
+// goes out of scope).
+template <typename T>
+static hipError_t upload(hh_scene s, std::vector<void*>& allocs, const std::vector<T>& v, T** out) {
+    HH_TRY(dalloc(allocs, v.size(), out));
+    if (!v.empty()) HH_TRY(hipMemcpyAsync(*out, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s->ctx->stream));
     return hipSuccess;
 }
+// Several host arrays laid out in one block: one allocation and one copy.
+struct TableBlob {
+    std::vector<unsigned char> bytes;
+    template <typename T>
+    size_t add(const std::vector<T>& v) {
+        const size_t at = (bytes.size() + 255) / 256 * 256;
+        bytes.resize(at + std::max<size_t>(v.size() * sizeof(T), 16));
+        if (!v.empty()) std::memcpy(bytes.data() + at, v.data(), v.size() * sizeof(T));
+        return at;
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Context
@@ -649,7 +705,7 @@ hh_status hh_scene_add_texture(hh_scene s, uint32_t w, uint32_t h, uint32_t form
     }
     s->textures.push_back(std::move(t));
     *out_id = (uint32_t)s->textures.size() - 1;
-    s->dirty = true;
+    s->edited(true, false);
     return HH_OK;
 }
 
@@ -660,7 +716,7 @@ hh_status hh_scene_add_material(hh_scene s, const hh_material_desc* d, uint32_t*
     for (int32_t t : tex) HH_ARG(t >= -1 && t < (int32_t)s->textures.size(), "material references an unknown texture");
     s->materials.push_back(*d);
     *out_id = (uint32_t)s->materials.size() - 1;
-    s->dirty = true;
+    s->edited(true, false);
     return HH_OK;
 }
 
@@ -687,7 +743,7 @@ hh_status hh_scene_add_mesh(hh_scene s, const hh_vertex* v, uint32_t nv, const u
     m.mats.assign(mats, mats + nm);
     s->meshes.push_back(std::move(m));
     *out_id = (uint32_t)s->meshes.size() - 1;
-    s->dirty = true;
+    s->edited(true, false);
     return HH_OK;
 }
 
@@ -700,7 +756,7 @@ hh_status hh_scene_add_instance(hh_scene s, const hh_instance_desc* d, uint32_t*
     for (int i = 0; i < 16; i++) HH_ARG(std::isfinite(d->model[i]) && std::isfinite(d->normal[i]), "non-finite transform");
     s->instances.push_back(*d);
     *out_id = (uint32_t)s->instances.size() - 1;
-    s->dirty = true;
+    s->edited(true, false);
     return HH_OK;
 }
 
@@ -710,7 +766,7 @@ hh_status hh_scene_set_instance_transform(hh_scene s, uint32_t i, const float mo
     for (int k = 0; k < 16; k++) HH_ARG(std::isfinite(model[k]) && std::isfinite(normal[k]), "non-finite transform");
     std::memcpy(s->instances[i].model, model, 64);
     std::memcpy(s->instances[i].normal, normal, 64);
-    s->dirty = true;
+    s->edited(false, false);
     return HH_OK;
 }
 
@@ -720,7 +776,7 @@ hh_status hh_scene_add_light(hh_scene s, const hh_light_desc* d, uint32_t* out_i
     if (s->lights.size() >= HH_MAX_SCENE_LIGHT_COUNT) return fail(HH_ERR_LIMIT_EXCEEDED, "too many lights");
     s->lights.push_back(*d);
     *out_id = (uint32_t)s->lights.size() - 1;
-    s->dirty = true;
+    s->edited(false, true);
     return HH_OK;
 }
 
@@ -734,7 +790,7 @@ hh_status hh_scene_set_ibl(hh_scene s, uint32_t size, const float* faces) {
         s->ibl.assign(faces, faces + size_t(6) * size * size * 4);
         s->ibl_size = size;
     }
-    s->dirty = true;
+    s->edited(false, true);
     return HH_OK;
 }
 
@@ -746,7 +802,158 @@ hh_status hh_scene_set_sky(hh_scene s, const hh_sky_params* p) {
     HH_ARG(p->equirect_width == 0 || (p->equirect_width >= 16 && p->equirect_width <= 16384 && p->equirect_width % 2 == 0),
            "equirect_width must be 0 or even in [16, 16384]");
     s->sky = *p;
-    s->dirty = true;
+    s->edited(false, true);
+    return HH_OK;
+}
+
+// The geometry of a scene: pools, triangle records and a BLAS per mesh
+// (mesh.cpp:46-117), textures. Replaces what an earlier commit built.
+static hh_status build_geometry(hh_scene s, const std::vector<uint32_t>& global_meshes, const std::vector<uint32_t>& vbase,
+                                const std::vector<uint32_t>& ibase, const std::vector<uint32_t>& mesh_tris, size_t nv,
+                                size_t ni, size_t ntri, const std::vector<int32_t>& tex_slots) {
+    hh_context ctx = s->ctx;
+    const int W = ctx->tune.bvh_width;
+    s->free_geometry();
+    auto& geo = s->geom;
+    const size_t node_bytes = W == 8 ? sizeof(WideNode<8>) : sizeof(WideNode<4>);
+    size_t node_cap = s->instances.size() + 2;
+    for (uint32_t t : mesh_tris) node_cap += t + 1;
+    unsigned char* nodes = nullptr;
+    HH_HIP(dalloc(geo.allocs, 5 * nv, &geo.vtx));
+    HH_HIP(dalloc(geo.allocs, ni, &geo.idx));
+    HH_HIP(dalloc(geo.allocs, node_cap * node_bytes, &nodes));
+    HH_HIP(dalloc(geo.allocs, ntri * 3, &geo.tris));
+    HH_HIP(dalloc(geo.allocs, ntri * 4, &geo.shade));
+    geo.nodes = nodes;
+    if (ctx->tune.bvh_compressed && W == 4) {
+        QNode4* q = nullptr;
+        HH_HIP(dalloc(geo.allocs, node_cap, &q));
+        geo.qnodes = q;
+    }
+    float4 *d_vtx = geo.vtx, *d_tris = geo.tris, *d_shade = geo.shade;
+    uint32_t* d_idx = geo.idx;
+    void* d_nodes = geo.nodes;
+    for (size_t g = 0; g < global_meshes.size(); g++) {
+        const MeshHost& me = s->meshes[global_meshes[g]];
+        if (!me.v.empty())
+            HH_HIP(hipMemcpyAsync((char*)d_vtx + size_t(vbase[g]) * sizeof(hh_vertex), me.v.data(), me.v.size() * sizeof(hh_vertex),
+                                  hipMemcpyHostToDevice, ctx->stream));
+        if (!me.idx.empty())
+            HH_HIP(hipMemcpyAsync(d_idx + ibase[g], me.idx.data(), me.idx.size() * 4, hipMemcpyHostToDevice, ctx->stream));
+    }
+    std::vector<uint32_t>& blas_root = geo.blas_root;
+    std::vector<float>& blas_box = geo.blas_box;
+    blas_root.assign(global_meshes.size(), 0u);
+    blas_box.assign(global_meshes.size() * 6, 0.0f);
+    // Per-triangle positions (3 float4: xyz + primitive index / geometry index
+    // and opaque bit in w) and shading records (4 float4, leaf order like the
+    // positions): (u0 v0 u1 v1) (u2 v2 n0.x n0.y) (n0.z n1.xyz) (n2.xyz 0), the
+    // vertex attributes the shading and the alpha test interpolate, in one
+    // line. Mesh g owns triangles tri_off[g]..; an empty mesh one inert
+    // triangle. Gathered on the GPU from the vertex and index pools; the host
+    // builder's copy of the positions is filled on the host.
+    const size_t G = global_meshes.size();
+    std::vector<uint32_t> tri_off(G + 1, 0);
+    for (size_t g = 0; g < G; g++) tri_off[g + 1] = tri_off[g] + mesh_tris[g];
+    auto geom_word = [&](const MeshHost& me, uint32_t gi) -> uint32_t {
+        const hh_material_desc& m = s->materials[me.mats[me.sm[gi].mat_idx]];
+        return gi | ((m.type == HH_MATERIAL_OPAQUE && !m.alpha_test) ? 0x80000000u : 0u);  // mesh.cpp:75-76
+    };
+    std::vector<SoupRange> soup_ranges;
+    for (size_t g = 0; g < G; g++) {
+        const MeshHost& me = s->meshes[global_meshes[g]];
+        uint32_t t = tri_off[g];
+        for (uint32_t gi = 0; gi < me.sm.size(); gi++) {
+            const hh_submesh& sm = me.sm[gi];
+            if (sm.index_count == 0) continue;
+            soup_ranges.push_back({t, ibase[g] + sm.base_index, vbase[g], geom_word(me, gi)});
+            t += sm.index_count / 3;
+        }
+        if (t == tri_off[g]) soup_ranges.push_back({t, kInertSoup, 0u, 0u});
+    }
+    std::vector<float4> soup;
+    if (ctx->tune.bvh_builder == 1) {   // the host builder reads the triangles
+        soup.assign(ntri * 3, make_float4(0.f, 0.f, 0.f, 0.f));
+        for (size_t g = 0; g < G; g++) {
+            const MeshHost& me = s->meshes[global_meshes[g]];
+            float4* ps = &soup[3 * size_t(tri_off[g])];
+            for (const hh_submesh& sm : me.sm)
+                for (uint32_t k = 0; k < sm.index_count; k++, ps++) {
+                    const float* p = me.v[me.idx[sm.base_index + k]].position;
+                    *ps = make_float4(p[0], p[1], p[2], 0.f);
+                }
+        }
+    }
+    float4* d_soup = nullptr;
+    float4* d_shade_soup = nullptr;
+    SoupRange* d_ranges = nullptr;
+    hipError_t e = hipMalloc(&d_soup, std::max<size_t>(ntri, 1) * 3 * sizeof(float4));
+    if (e == hipSuccess) e = hipMalloc(&d_shade_soup, std::max<size_t>(ntri, 1) * 4 * sizeof(float4));
+    if (e == hipSuccess) e = hipMalloc(&d_ranges, std::max<size_t>(soup_ranges.size(), 1) * sizeof(SoupRange));
+    if (e == hipSuccess && !soup_ranges.empty())
+        e = hipMemcpyAsync(d_ranges, soup_ranges.data(), soup_ranges.size() * sizeof(SoupRange), hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess)
+        e = launch_soup(ctx->stream, d_ranges, (uint32_t)soup_ranges.size(), (uint32_t)ntri, d_vtx, d_idx, d_soup, d_shade_soup);
+    hh_status st = HH_OK;
+    uint32_t node_base = 0, tri_base = 0;
+    if (e != hipSuccess) {
+        st = hip_fail(e, "triangle records");
+    } else if (G == 0) {
+        // no meshes: no BLAS
+    } else if (ctx->tune.bvh_builder == 3) {
+        // every mesh's tree on the GPU together
+        std::vector<int2> ranges(G);
+        for (size_t g = 0; g < G; g++) {
+            ranges[g] = make_int2((int)tri_off[g], (int)mesh_tris[g]);
+            blas_root[g] = (uint32_t)g;
+        }
+        e = build_blas_forest(ctx->stream, W, ctx->tune.leaf_size, ranges, (uint32_t)ntri, d_soup, d_tris, d_shade_soup,
+                              d_shade, d_nodes, 0, ctx->bs, &node_base, blas_box.data());
+        if (e != hipSuccess) st = hip_fail(e, "BLAS build");
+        tri_base = (uint32_t)ntri;
+    } else {
+        for (size_t g = 0; g < G; g++) {
+            const uint32_t n = mesh_tris[g], off = tri_off[g];
+            uint32_t nn = 0;
+            e = build_blas(ctx->stream, W, ctx->tune.leaf_size, n, d_soup + 3 * size_t(off), d_tris,
+                           d_shade_soup + 4 * size_t(off), d_shade,
+                           ctx->tune.bvh_builder == 1 ? soup.data() + 3 * size_t(off) : nullptr, tri_base, d_nodes, node_base,
+                           ctx->bs, &nn, &blas_box[g * 6], ctx->tune.bvh_builder == 2, false);
+            if (e != hipSuccess) {
+                st = hip_fail(e, "BLAS build");
+                break;
+            }
+            blas_root[g] = node_base;
+            node_base += nn;
+            tri_base += n;
+        }
+    }
+    (void)hipStreamSynchronize(ctx->stream);
+    if (d_soup) (void)hipFree(d_soup);
+    if (d_shade_soup) (void)hipFree(d_shade_soup);
+    if (d_ranges) (void)hipFree(d_ranges);
+    if (st != HH_OK) return st;
+    // textures
+    std::vector<TexDesc> tdesc;
+    std::vector<float4> texels;
+    for (int32_t tid : tex_slots) {
+        const TexHost& t = s->textures[tid];
+        TexDesc d{(uint32_t)texels.size(), t.w, t.h, 0};
+        tdesc.push_back(d);
+        for (size_t i = 0; i < size_t(t.w) * t.h; i++)
+            texels.push_back(make_float4(t.texels[i * 4], t.texels[i * 4 + 1], t.texels[i * 4 + 2], t.texels[i * 4 + 3]));
+    }
+    HH_HIP(upload(s, geo.allocs, vbase, &geo.vbase));
+    HH_HIP(upload(s, geo.allocs, ibase, &geo.ibase));
+    HH_HIP(upload(s, geo.allocs, tdesc, &geo.tex));
+    HH_HIP(upload(s, geo.allocs, texels, &geo.texels));
+    HH_HIP(hipStreamSynchronize(ctx->stream));
+    geo.num_nodes = node_base;
+    geo.num_tris = tri_base;
+    geo.width = W;
+    geo.builder = ctx->tune.bvh_builder;
+    geo.compressed = ctx->tune.bvh_compressed;
+    geo.built = true;
     return HH_OK;
 }
 
@@ -755,9 +962,12 @@ hh_status hh_scene_commit(hh_scene s) {
     hh_context ctx = s->ctx;
     HH_HIP(hipSetDevice(ctx->device));
     HH_HIP(hipStreamSynchronize(ctx->stream));
-    ctx->drop_graphs();
-    s->free_device();
+    s->committed = false;
     const int W = ctx->tune.bvh_width;
+    // not reused under another BVH tuning
+    if (s->geom.width != W || s->geom.builder != ctx->tune.bvh_builder || s->geom.compressed != ctx->tune.bvh_compressed)
+        s->geom.built = false;
+    const bool new_geom = !s->geom.built;
     // ---- packing (scene.cpp:915-1311) -------------------------------------
     std::vector<MaterialData> mat_data;
     std::vector<int32_t> tex_slots;
@@ -905,120 +1115,17 @@ hh_status hh_scene_commit(hh_scene s) {
         ntri += mesh_tris[g];
     }
     if (ntri >= kLeafStartMask) return fail(HH_ERR_LIMIT_EXCEEDED, "too many triangles (%zu)", ntri);
-    float4* d_vtx = nullptr;
-    uint32_t* d_idx = nullptr;
-    HH_HIP(dalloc(s, nv * sizeof(hh_vertex), (void**)&d_vtx));
-    HH_HIP(dalloc(s, ni * 4, (void**)&d_idx));
-    for (size_t g = 0; g < global_meshes.size(); g++) {
-        const MeshHost& me = s->meshes[global_meshes[g]];
-        if (!me.v.empty())
-            HH_HIP(hipMemcpyAsync((char*)d_vtx + size_t(vbase[g]) * sizeof(hh_vertex), me.v.data(), me.v.size() * sizeof(hh_vertex),
-                                  hipMemcpyHostToDevice, ctx->stream));
-        if (!me.idx.empty())
-            HH_HIP(hipMemcpyAsync(d_idx + ibase[g], me.idx.data(), me.idx.size() * 4, hipMemcpyHostToDevice, ctx->stream));
-    }
-    // ---- BLAS per mesh (mesh.cpp:46-117) ------------------------------------
+    auto& geo = s->geom;
     const size_t node_bytes = W == 8 ? sizeof(WideNode<8>) : sizeof(WideNode<4>);
-    size_t node_cap = s->instances.size() + 2;
-    for (uint32_t t : mesh_tris) node_cap += t + 1;
-    void* d_nodes = nullptr;
-    float4* d_tris = nullptr;
-    float4* d_shade = nullptr;
-    HH_HIP(dalloc(s, node_cap * node_bytes, &d_nodes));
-    HH_HIP(dalloc(s, ntri * 3 * sizeof(float4), (void**)&d_tris));
-    HH_HIP(dalloc(s, ntri * 4 * sizeof(float4), (void**)&d_shade));
-    std::vector<uint32_t> blas_root(global_meshes.size());
-    std::vector<float> blas_box(global_meshes.size() * 6);
-    uint32_t node_base = 0, tri_base = 0;
-    // Per-triangle positions (3 float4: xyz + primitive index / geometry index
-    // and opaque bit in w) and shading records (4 float4, leaf order like the
-    // positions): (u0 v0 u1 v1) (u2 v2 n0.x n0.y) (n0.z n1.xyz) (n2.xyz 0), the
-    // vertex attributes the shading and the alpha test interpolate, in one
-    // line. Mesh g owns triangles tri_off[g]..; an empty mesh one inert
-    // triangle. Gathered on the GPU from the vertex and index pools; the host
-    // builder's copy of the positions is filled on the host.
-    const size_t G = global_meshes.size();
-    std::vector<uint32_t> tri_off(G + 1, 0);
-    for (size_t g = 0; g < G; g++) tri_off[g + 1] = tri_off[g] + mesh_tris[g];
-    auto geom_word = [&](const MeshHost& me, uint32_t gi) -> uint32_t {
-        const hh_material_desc& m = s->materials[me.mats[me.sm[gi].mat_idx]];
-        return gi | ((m.type == HH_MATERIAL_OPAQUE && !m.alpha_test) ? 0x80000000u : 0u);  // mesh.cpp:75-76
-    };
-    std::vector<SoupRange> soup_ranges;
-    for (size_t g = 0; g < G; g++) {
-        const MeshHost& me = s->meshes[global_meshes[g]];
-        uint32_t t = tri_off[g];
-        for (uint32_t gi = 0; gi < me.sm.size(); gi++) {
-            const hh_submesh& sm = me.sm[gi];
-            if (sm.index_count == 0) continue;
-            soup_ranges.push_back({t, ibase[g] + sm.base_index, vbase[g], geom_word(me, gi)});
-            t += sm.index_count / 3;
-        }
-        if (t == tri_off[g]) soup_ranges.push_back({t, kInertSoup, 0u, 0u});
-    }
-    std::vector<float4> soup;
-    if (ctx->tune.bvh_builder == 1) {   // the host builder reads the triangles
-        soup.assign(ntri * 3, make_float4(0.f, 0.f, 0.f, 0.f));
-        for (size_t g = 0; g < G; g++) {
-            const MeshHost& me = s->meshes[global_meshes[g]];
-            float4* ps = &soup[3 * size_t(tri_off[g])];
-            for (const hh_submesh& sm : me.sm)
-                for (uint32_t k = 0; k < sm.index_count; k++, ps++) {
-                    const float* p = me.v[me.idx[sm.base_index + k]].position;
-                    *ps = make_float4(p[0], p[1], p[2], 0.f);
-                }
-        }
-    }
-    float4* d_soup = nullptr;
-    float4* d_shade_soup = nullptr;
-    SoupRange* d_ranges = nullptr;
-    hipError_t e = hipMalloc(&d_soup, std::max<size_t>(ntri, 1) * 3 * sizeof(float4));
-    if (e == hipSuccess) e = hipMalloc(&d_shade_soup, std::max<size_t>(ntri, 1) * 4 * sizeof(float4));
-    if (e == hipSuccess) e = hipMalloc(&d_ranges, std::max<size_t>(soup_ranges.size(), 1) * sizeof(SoupRange));
-    if (e == hipSuccess && !soup_ranges.empty())
-        e = hipMemcpyAsync(d_ranges, soup_ranges.data(), soup_ranges.size() * sizeof(SoupRange), hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess)
-        e = launch_soup(ctx->stream, d_ranges, (uint32_t)soup_ranges.size(), (uint32_t)ntri, d_vtx, d_idx, d_soup, d_shade_soup);
     hh_status st = HH_OK;
-    if (e != hipSuccess) {
-        st = hip_fail(e, "triangle records");
-    } else if (G == 0) {
-        // no meshes: no BLAS
-    } else if (ctx->tune.bvh_builder == 3) {
-        // every mesh's tree on the GPU together
-        std::vector<int2> ranges(G);
-        for (size_t g = 0; g < G; g++) {
-            ranges[g] = make_int2((int)tri_off[g], (int)mesh_tris[g]);
-            blas_root[g] = (uint32_t)g;
-        }
-        e = build_blas_forest(ctx->stream, W, ctx->tune.leaf_size, ranges, (uint32_t)ntri, d_soup, d_tris, d_shade_soup,
-                              d_shade, d_nodes, 0, ctx->bs, &node_base, blas_box.data());
-        if (e != hipSuccess) st = hip_fail(e, "BLAS build");
-        tri_base = (uint32_t)ntri;
-    } else {
-        for (size_t g = 0; g < G; g++) {
-            const uint32_t n = mesh_tris[g], off = tri_off[g];
-            uint32_t nn = 0;
-            e = build_blas(ctx->stream, W, ctx->tune.leaf_size, n, d_soup + 3 * size_t(off), d_tris,
-                           d_shade_soup + 4 * size_t(off), d_shade,
-                           ctx->tune.bvh_builder == 1 ? soup.data() + 3 * size_t(off) : nullptr, tri_base, d_nodes, node_base,
-                           ctx->bs, &nn, &blas_box[g * 6], ctx->tune.bvh_builder == 2, false);
-            if (e != hipSuccess) {
-                st = hip_fail(e, "BLAS build");
-                break;
-            }
-            blas_root[g] = node_base;
-            node_base += nn;
-            tri_base += n;
-        }
-    }
-    (void)hipStreamSynchronize(ctx->stream);
-    if (d_soup) (void)hipFree(d_soup);
-    if (d_shade_soup) (void)hipFree(d_shade_soup);
-    if (d_ranges) (void)hipFree(d_ranges);
+    if (new_geom) st = build_geometry(s, global_meshes, vbase, ibase, mesh_tris, nv, ni, ntri, tex_slots);
     if (st != HH_OK) return st;
-    s->bvh_stats[0] = node_base;
-    s->bvh_stats[1] = tri_base;
+    void* d_nodes = geo.nodes;
+    const std::vector<uint32_t>& blas_root = geo.blas_root;
+    const std::vector<float>& blas_box = geo.blas_box;
+    const uint32_t node_base = geo.num_nodes;
+    s->bvh_stats[0] = geo.num_nodes;
+    s->bvh_stats[1] = geo.num_tris;
     // ---- TLAS over instances (renderer.cpp:113-181) ---------------------------
     std::vector<InstTrav> trav(s->instances.size());
     std::vector<float> ilo(s->instances.size() * 3), ihi(s->instances.size() * 3);
@@ -1088,26 +1195,15 @@ hh_status hh_scene_commit(hh_scene s) {
     }
     s->bvh_stats[2] = tlas_nodes;
     s->bvh_stats[3] = global_meshes.size();
-    // Optional 64-B quantized BVH4 nodes (same topology and indices).
+    // Optional 64-B quantized BVH4 nodes (same topology and indices): all of
+    // them with new geometry, else the TLAS's.
     int layout = W;
-    if (ctx->tune.bvh_compressed && W == 4) {
-        void* q = nullptr;
-        const uint32_t total_nodes = node_base + tlas_nodes;
-        HH_HIP(dalloc(s, size_t(total_nodes) * sizeof(QNode4), &q));
-        HH_HIP(quantize_bvh4(ctx->stream, d_nodes, q, total_nodes));
-        HH_HIP(hipStreamSynchronize(ctx->stream));
-        d_nodes = q;
+    if (geo.qnodes) {
+        const uint32_t first = new_geom ? 0u : node_base;
+        HH_HIP(quantize_bvh4(ctx->stream, (char*)d_nodes + size_t(first) * node_bytes, (QNode4*)geo.qnodes + first,
+                             node_base + tlas_nodes - first));
+        d_nodes = geo.qnodes;
         layout = kLayoutQ4;
-    }
-    // ---- textures --------------------------------------------------------------
-    std::vector<TexDesc> tdesc;
-    std::vector<float4> texels;
-    for (int32_t tid : tex_slots) {
-        const TexHost& t = s->textures[tid];
-        TexDesc d{(uint32_t)texels.size(), t.w, t.h, 0};
-        tdesc.push_back(d);
-        for (size_t i = 0; i < size_t(t.w) * t.h; i++)
-            texels.push_back(make_float4(t.texels[i * 4], t.texels[i * 4 + 1], t.texels[i * 4 + 2], t.texels[i * 4 + 3]));
     }
     // ---- power-proportional emitters (HH_FLAG_LIGHT_POWER): every emissive
     // triangle of every instance in world space; selection probability
@@ -1169,23 +1265,27 @@ hh_status hh_scene_commit(hh_scene s) {
         }
     }
     // ---- environment: IBL, sky (directional light), or the black 2x2 default -----
-    uint32_t env_size;
-    float4* d_env = nullptr;
-    uint16_t* d_env_eq = nullptr;
+    if (!s->env.built) s->free_environment();
+    auto& en = s->env;
+    uint32_t& env_size = en.size;
+    float4*& d_env = en.cube;
+    uint16_t*& d_env_eq = en.eq;
     const uint32_t eq_w = (!has_ibl && n_dir > 0) ? s->sky.equirect_width : 0u;
-    if (eq_w > 0) {
+    if (en.built) {
+        // unchanged since it was made
+    } else if (eq_w > 0) {
         // extension: the sky as an equirectangular RGBA16F map (no cube)
         float sd[3] = {-sun->forward[0], -sun->forward[1], -sun->forward[2]};
         sky_coefficients(s->sky.turbidity, s->sky.albedo, s->sky.normalized_sun_y, sd, s->sky_coef);
         HH_HIP(hipMemcpyAsync(ctx->d_coef, s->sky_coef, sizeof(s->sky_coef), hipMemcpyHostToDevice, ctx->stream));
-        HH_HIP(dalloc(s, size_t(eq_w) * (eq_w / 2) * 4 * sizeof(uint16_t), (void**)&d_env_eq));
+        HH_HIP(dalloc(en.allocs, size_t(eq_w) * (eq_w / 2) * 4, &d_env_eq));
         HH_HIP(launch_sky_bake_equirect(ctx->stream, d_env_eq, eq_w, ctx->d_coef, sd));
         env_size = 2;
-        HH_HIP(dalloc(s, 6 * 4 * sizeof(float4), (void**)&d_env));
+        HH_HIP(dalloc(en.allocs, 24, &d_env));
         HH_HIP(launch_fill_f4(ctx->stream, d_env, make_float4(0.f, 0.f, 0.f, 0.f), 24));
     } else if (has_ibl) {
         env_size = s->ibl_size;
-        HH_HIP(dalloc(s, size_t(6) * env_size * env_size * sizeof(float4), (void**)&d_env));
+        HH_HIP(dalloc(en.allocs, size_t(6) * env_size * env_size, &d_env));
         HH_HIP(hipMemcpyAsync(d_env, s->ibl.data(), size_t(6) * env_size * env_size * sizeof(float4), hipMemcpyHostToDevice,
                               ctx->stream));
     } else if (n_dir > 0) {
@@ -1193,20 +1293,25 @@ hh_status hh_scene_commit(hh_scene s) {
         float sd[3] = {-sun->forward[0], -sun->forward[1], -sun->forward[2]};
         sky_coefficients(s->sky.turbidity, s->sky.albedo, s->sky.normalized_sun_y, sd, s->sky_coef);
         HH_HIP(hipMemcpyAsync(ctx->d_coef, s->sky_coef, sizeof(s->sky_coef), hipMemcpyHostToDevice, ctx->stream));
-        HH_HIP(dalloc(s, size_t(6) * env_size * env_size * sizeof(float4), (void**)&d_env));
+        HH_HIP(dalloc(en.allocs, size_t(6) * env_size * env_size, &d_env));
         HH_HIP(launch_sky_bake(ctx->stream, d_env, env_size, ctx->d_coef, sd));
     } else {
         env_size = 2;
-        HH_HIP(dalloc(s, 6 * 4 * sizeof(float4), (void**)&d_env));
+        HH_HIP(dalloc(en.allocs, 24, &d_env));
         HH_HIP(launch_fill_f4(ctx->stream, d_env, make_float4(0.f, 0.f, 0.f, 0.f), 24));
     }
+    en.eq_w = eq_w;
     // ---- upload tables --------------------------------------------------------
     SceneGPU g{};
     g.nodes = d_nodes;
-    g.tris = d_tris;
-    g.shade = d_shade;
-    g.vtx = d_vtx;
-    g.idx = d_idx;
+    g.tris = geo.tris;
+    g.shade = geo.shade;
+    g.vtx = geo.vtx;
+    g.idx = geo.idx;
+    g.vbase = geo.vbase;
+    g.ibase = geo.ibase;
+    g.tex = geo.tex;
+    g.texels = geo.texels;
     g.env = d_env;
     g.env_size = env_size;
     g.num_lights = num_lights;
@@ -1215,29 +1320,38 @@ hh_status hh_scene_commit(hh_scene s) {
     g.env_eq_w = eq_w;
     g.num_area = (uint32_t)area.size();
     g.num_emit = (uint32_t)emit_cdf.size();
-    if (!emit_cdf.empty()) {
-        HH_HIP(upload(s, emit_tri, (float4**)&g.emit_tri));
-        HH_HIP(upload(s, emit_le, (float4**)&g.emit_le));
-        HH_HIP(upload(s, emit_cdf, (float**)&g.emit_cdf));
-    }
     g.bvh_width = (uint32_t)layout;
-    {
-        const std::vector<unsigned long long> zeros(kNumFaults, 0ull);
-        HH_HIP(upload(s, zeros, &g.faults));
+    TableBlob blob;
+    const std::vector<unsigned long long> zeros(kNumFaults, 0ull);
+    const size_t o_faults = blob.add(zeros), o_trav = blob.add(trav), o_inst = blob.add(inst_data), o_mats = blob.add(mat_data),
+                 o_lights = blob.add(lights), o_off = blob.add(submesh_off), o_info = blob.add(submesh_info),
+                 o_etri = blob.add(emit_tri), o_ele = blob.add(emit_le), o_ecdf = blob.add(emit_cdf),
+                 o_gpu = blob.add(std::vector<SceneGPU>{g});
+    if (blob.bytes.size() > s->tables_cap) {
+        if (s->tables) HH_HIP(hipFree(s->tables));
+        s->tables = nullptr;
+        s->tables_cap = 0;
+        HH_HIP(hipMalloc((void**)&s->tables, blob.bytes.size()));
+        s->tables_cap = blob.bytes.size();
     }
-    HH_HIP(upload(s, trav, (InstTrav**)&g.inst_trav));
-    HH_HIP(upload(s, inst_data, (InstanceData**)&g.inst));
-    HH_HIP(upload(s, mat_data, (MaterialData**)&g.mats));
-    HH_HIP(upload(s, lights, (LightData**)&g.lights));
-    HH_HIP(upload(s, submesh_off, (uint32_t**)&g.submesh_off));
-    HH_HIP(upload(s, submesh_info, (uint2**)&g.submesh_info));
-    HH_HIP(upload(s, vbase, (uint32_t**)&g.vbase));
-    HH_HIP(upload(s, ibase, (uint32_t**)&g.ibase));
-    HH_HIP(upload(s, tdesc, (TexDesc**)&g.tex));
-    HH_HIP(upload(s, texels, (float4**)&g.texels));
-    std::vector<SceneGPU> one{g};
-    HH_HIP(upload(s, one, &s->d_gpu));
+    unsigned char* const base = s->tables;
+    g.faults = (unsigned long long*)(base + o_faults);
+    g.inst_trav = (InstTrav*)(base + o_trav);
+    g.inst = (InstanceData*)(base + o_inst);
+    g.mats = (MaterialData*)(base + o_mats);
+    g.lights = (LightData*)(base + o_lights);
+    g.submesh_off = (uint32_t*)(base + o_off);
+    g.submesh_info = (uint2*)(base + o_info);
+    if (!emit_cdf.empty()) {
+        g.emit_tri = (float4*)(base + o_etri);
+        g.emit_le = (float4*)(base + o_ele);
+        g.emit_cdf = (float*)(base + o_ecdf);
+    }
+    std::memcpy(blob.bytes.data() + o_gpu, &g, sizeof(g));
+    s->d_gpu = (SceneGPU*)(base + o_gpu);
+    HH_HIP(hipMemcpyAsync(base, blob.bytes.data(), blob.bytes.size(), hipMemcpyHostToDevice, ctx->stream));
     HH_HIP(hipStreamSynchronize(ctx->stream));
+    en.built = true;
     s->gpu = g;
     s->committed = true;
     s->dirty = false;
@@ -1510,7 +1624,7 @@ static hipError_t upload_tables(hh_context ctx, const std::vector<SceneGPU>& sce
 }
 
 static hh_status run_frame(hh_context ctx, const std::vector<SceneGPU>& scenes, const std::vector<ViewGPU>& views,
-                           uint32_t total, uint32_t max_bounces, bool mega, const std::string& key_extra) {
+                           uint32_t total, uint32_t max_bounces, bool mega) {
     HH_HIP(ensure_tables(ctx, (uint32_t)scenes.size(), (uint32_t)views.size()));
     uint32_t cap_before = ctx->wf.capacity;
     uint32_t* spill_before = ctx->wf.spill;
@@ -1543,14 +1657,21 @@ static hh_status run_frame(hh_context ctx, const std::vector<SceneGPU>& scenes, 
                             max_bounces, ctx->wf, mega));
         return HH_OK;
     }
-    // The launch sequence depends on the view geometry (tile sizes, spp) and
-    // the bounce count, not on camera or frame index (read from d_views).
-    std::string key = key_extra + "|" + std::to_string(total) + "|" + std::to_string(max_bounces) + "|" + std::to_string(mega) +
-                      "|" + std::to_string(views.size());
+    // The launch sequence depends on the node layout, the bounce count and the
+    // views' geometry (tile sizes, spp, which of them share a scene); scenes,
+    // surfaces, cameras and frame indices are read from the scene and view
+    // tables, so a graph serves every scene of its shape and outlives commits.
+    std::string key = std::to_string(scenes[0].bvh_width) + "|" + std::to_string(total) + "|" + std::to_string(max_bounces) + "|" +
+                      std::to_string(mega);
     for (const ViewGPU& v : views)
-        key += "|" + std::to_string(v.tile_w) + "x" + std::to_string(v.tile_h) + "s" + std::to_string(v.spp);
+        key += "|" + std::to_string(v.tile_w) + "x" + std::to_string(v.tile_h) + "s" + std::to_string(v.spp) + "@" +
+               std::to_string(v.scene);
     auto it = ctx->graphs.find(key);
     if (it == ctx->graphs.end()) {
+        if (ctx->graphs.size() >= kMaxGraphs) {   // shapes keep changing: start over (the frames in flight end first)
+            HH_HIP(hipStreamSynchronize(ctx->stream));
+            ctx->drop_graphs();
+        }
         GraphEntry ge;
         HH_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
         hipError_t e = launch_frame(cfg, ctx->d_scene_table, scenes.data(), ctx->d_views, views.data(), (uint32_t)views.size(), total,
@@ -1685,8 +1806,7 @@ hh_status hh_integrator_render_frames(hh_integrator it, hh_scene scene, const hh
         v.accum = out->d;
         v.aux = out->aux;
         std::vector<ViewGPU> views{v};
-        st = run_frame(ctx, scenes, views, v.tile_w * v.tile_h * chunk, it->s.max_ray_bounces, mega,
-                       std::to_string(scene->generation) + "|" + std::to_string((uintptr_t)out->d));
+        st = run_frame(ctx, scenes, views, v.tile_w * v.tile_h * chunk, it->s.max_ray_bounces, mega);
         if (st != HH_OK) return st;
         it->num_acc += chunk;
         launched += chunk;
@@ -1751,12 +1871,10 @@ hh_status hh_render_batch(hh_context ctx, const hh_view* views, uint32_t n) {
     }
     std::map<hh_scene, uint32_t> scene_index;
     std::vector<SceneGPU> scenes;
-    std::string key = "batch";
     for (uint32_t i = 0; i < n; i++)
         if (!scene_index.count(views[i].scene)) {
             scene_index[views[i].scene] = (uint32_t)scenes.size();
             scenes.push_back(views[i].scene->gpu);
-            key += "|" + std::to_string(views[i].scene->generation);
         }
     for (auto& sg : scenes) HH_ARG(sg.bvh_width == scenes[0].bvh_width, "scenes of one batch must share the BVH width");
     unsigned long long zero[2] = {0, 0};
@@ -1795,9 +1913,7 @@ hh_status hh_render_batch(hh_context ctx, const hh_view* views, uint32_t n) {
             vg.push_back(v);
         }
         HH_ARG(total <= kMaxPathSlots, "batch too large");
-        std::string k = key;
-        for (uint32_t i = 0; i < n; i++) k += "|" + std::to_string((uintptr_t)views[i].surface->d);
-        hh_status st = run_frame(ctx, scenes, vg, (uint32_t)total, maxb, false, k);
+        hh_status st = run_frame(ctx, scenes, vg, (uint32_t)total, maxb, false);
         if (st != HH_OK) return st;
     }
     return HH_OK;
