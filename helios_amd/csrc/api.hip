@@ -2172,12 +2172,11 @@ hh_status hh_render_output_buffer(hh_scene s, const hh_camera* cam, uint32_t whi
     HH_ARG(out->ctx == ctx, "surface belongs to another context");
     HH_HIP(hipSetDevice(ctx->device));
     const uint32_t w = out->w, h = out->h;
-    const size_t n = size_t(w) * h;
     HH_HIP(ensure_dbg(ctx, sizeof(ViewGPU)));
     ViewGPU* d_view = (ViewGPU*)ctx->dbg;
     ViewGPU v = make_view(*cam, w, h);
     HH_HIP(hipMemcpyAsync(d_view, &v, sizeof(v), hipMemcpyHostToDevice, ctx->stream));
-    HH_HIP(ensure_spill_keep_graphs(ctx, (n + 255) / 256 * 256));
+    HH_HIP(ensure_spill_keep_graphs(ctx, size_t(output_buffer_blocks(ctx->num_cu, w, h)) * 256));
     const double fn = cam->far_plane, nn = cam->near_plane;
     const float near_d = (float)(2.0 * fn * nn / (fn + nn));
     LaunchCfg cfg{ctx->stream, ctx->num_cu, ctx->tune};

@@ -225,6 +225,8 @@ hipError_t launch_pack_hits(hipStream_t stream, const float4* d_hit, const uint3
                             void* d_out);
 hipError_t launch_primary_hits(const LaunchCfg& cfg, const SceneGPU* d_scene, const SceneGPU& h_scene, const ViewGPU* d_view,
                                uint32_t w, uint32_t h, uint32_t frame, float4* d_hit, uint32_t* d_hit_ids, uint32_t* spill);
+// Workgroups (of 256 threads, each with a spill column) launch_output_buffer takes.
+uint32_t output_buffer_blocks(int num_cu, uint32_t w, uint32_t h);
 hipError_t launch_output_buffer(const LaunchCfg& cfg, const SceneGPU* d_scene, const SceneGPU& h_scene, const ViewGPU* d_view,
                                 uint32_t w, uint32_t h, float near_d, float far_d, uint32_t which, float4* out, uint32_t* spill);
 hipError_t launch_ray_debug(const LaunchCfg& cfg, const SceneGPU* d_scene, const SceneGPU& h_scene, const ViewGPU* d_view,
