@@ -2376,7 +2376,7 @@ hh_status hh_denoiser_forward(hh_denoiser d, const float* feats, uint32_t n, uin
     hh_status s = dn_stage(d, feats, nullptr, n, h, w, false);
     if (s != HH_OK) return s;
     hipStream_t st = d->ctx->stream;
-    HH_HIP(d->net.forward(st, nullptr, h, w));
+    HH_HIP(d->net.forward(st, nullptr, h, w, false));
     const uint32_t Hp = d->net.H, Wp = d->net.W;
     std::vector<float> o((size_t)n * Hp * Wp * 4);
     HH_HIP(hipMemcpyAsync(o.data(), d->net.out, o.size() * 4, hipMemcpyDeviceToHost, st));
@@ -2395,7 +2395,7 @@ hh_status hh_denoiser_loss_grad(hh_denoiser d, const float* feats, const float* 
     hh_status s = dn_stage(d, feats, target, n, h, w, true);
     if (s != HH_OK) return s;
     hipStream_t st = d->ctx->stream;
-    HH_HIP(d->net.forward(st, nullptr, h, w));
+    HH_HIP(d->net.forward(st, nullptr, h, w, true));
     HH_HIP(d->net.loss_and_backward(st, d->d_target, h, w, d->loss_kind));
     float l = 0.0f;
     HH_HIP(hipMemcpyAsync(&l, d->net.loss, 4, hipMemcpyDeviceToHost, st));
@@ -2432,7 +2432,7 @@ hh_status hh_denoise(hh_denoiser d, hh_surface in, uint32_t num_frames, hh_surfa
     HH_HIP(d->net.ensure(1, pad8(in->h), pad8(in->w), false));
     const uint32_t held = num_frames >= 2 ? num_frames - 1 : 1;
     HH_HIP(d->net.pack(st, nullptr, in->d, in->aux, held, in->h, in->w));
-    HH_HIP(d->net.forward(st, out->d, in->h, in->w));
+    HH_HIP(d->net.forward(st, out->d, in->h, in->w, false));
     return HH_OK;
 }
 

@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "internal.hpp"
 
@@ -37,7 +38,20 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
-enum Epi { EPI_BIAS_RELU = 0, EPI_MASK = 1, EPI_F32 = 2 };
+// What a convolution does with its sums: bias + ReLU -> BF16 (also 2x2 averaged
+// into `pool`, or through the 1x1 head instead of being stored), times a ReLU
+// mask -> BF16, or FP32. EPI_SPLIT is EPI_BIAS_RELU with another order of the
+// sums (see k_conv3x3).
+enum Epi { EPI_BIAS_RELU = 0, EPI_MASK = 1, EPI_F32 = 2, EPI_POOL = 3, EPI_HEAD = 4, EPI_SPLIT = 5 };
+struct ConvExtra {
+    __bf16* pool;              // EPI_POOL: half-resolution average
+    const __bf16* wh;          // EPI_HEAD: head weights (3, 32) and bias,
+    const float* bh;
+    const float4* resid;       // the input's log radiance,
+    float4* out;               // the network output in log space (when set)
+    float4* surface;           // and the h x w surface (when set)
+    uint32_t h, w;
+};
 
 __device__ inline bf16x8 zero8() {
     bf16x8 z;
@@ -48,174 +62,437 @@ __device__ inline bf16x8 zero8() {
 
 // ---------------------------------------------------------------------------
 // 3x3 convolution (forward, and the input gradient with flipped weights).
-// A workgroup of kConvRows waves computes kConvRows rows x TW pixels
-// (TW = 16 NT) of all COUT channels. Input channels are taken 32 at a time:
-// the (kConvRows + 2) x (TW + 2) halo tile of those channels is staged in LDS once
-// (coalesced 16-byte loads, zero outside the image and beyond CT; the
-// upsample + concat of the decoder is resolved here), then all 9 taps read
-// their B operands from LDS. The K order is (channel group, tap, channel):
-// the same products as the K order of the weights, summed in another order.
-// (Against one wave loading its B operands straight from global memory per
-// tap, staging the tile cut a 1080p forward pass from 1.45 to 1.21 ms.)
-constexpr int kConvRows = 4;              // output rows per workgroup, one wave each
-constexpr int kConvThreads = 64 * kConvRows;
-// Waves per SIMD the LDS of one workgroup (halo tile + staged weights) allows
-// on a 160 KB CU, one wave per SIMD per workgroup: the register budget is
-// held to it, so registers never cost a workgroup that the LDS would admit.
-// (Wider outputs, which read their weights from global memory, keep the
-// compiler's own budget.)
-constexpr int conv_waves(int cout) {
-    if (cout > 96) return 1;
-    const int tile = (kConvRows + 2) * (16 * 4 + 2) * 4 * 16;
-    const int wts = 9 * cout * 5 * 16;
-    const int w = 163840 / (tile + wts);
-    return w < 1 ? 1 : (w > 8 ? 8 : w);
+// A workgroup of four waves computes tiles of output rows x pixels of CB output
+// channels (gridDim.y slices of them). Input channels are taken 32 at a time:
+// the halo tile of those channels and their weights are staged in LDS (16-byte
+// loads, zero outside the image and beyond CT; the upsample + concat of the
+// decoder is resolved here), then all 9 taps read their operands from LDS. The
+// K order is (channel group, tap, channel), whatever the tile.
+//
+// A wave holds R rows x 16 NT pixels x CB channels of accumulators and keeps
+// the weights of a tap row in registers: per 9 R NT MT MFMAs of a group it
+// reads 9 (MT + R NT) fragments from LDS.
+//
+// EPI_SPLIT (the 48^ + 32 -> 32 decoder layer in inference): groups of one
+// source each, and the order (group, horizontal tap, vertical tap, channel),
+// which reads an input row once for up to three output rows, 9 MT +
+// 3 (R + 2) NT fragments: 156 -> 128 us at 1920 x 1080. The other layers gain
+// nothing from it (632 us in all with it everywhere, 641 here); training
+// keeps one order of the sums throughout.
+//
+// What bounds it is the vector instructions around the MFMAs: with the places
+// of a tile's chunks divided out of the thread number and checked per lane, a
+// tile of the 32 -> 32 layer took 650 of them per wave beside 72 MFMAs, and
+// prefetching or fusing gained nothing. So a pass of the staging takes a fixed
+// column per thread and a row per pass, whose address and range check are the
+// wave's (a buffer descriptor, of length zero for a row outside); workgroups
+// are persistent and keep the weights of a single-group layer, and load the
+// next group or tile during the MFMAs. 2x2 pooling and the 1x1 head are done
+// on the accumulators: their activations need not be read again (nor, for the
+// head in inference, written). 1920 x 1080, one state kept: 867 -> 641 us for
+// the network (32 -> 32 at full resolution 77 -> 64 us with pooling, its
+// activations' copy time 58; the 48^ + 32 -> 32 decoder layer 180 -> 128).
+// Two workgroups per resident slot instead of one: 689 against 668; a tile per
+// workgroup: 718.
+//
+// Large images: tiles 64 pixels wide, whose halo is 1.5 (1.25) times the tile.
+// Eight rows (R = 4) only for 32 channels of several groups, where the staged
+// weights and the fragment reads of LDS weigh most: 174 -> 128 us; with 48
+// channels they spill (69 -> 100 us), and single-group layers are bound by
+// memory and want the third workgroup per CU.
+// Images with too few such tiles to fill the chip: 4 rows x 16 pixels and
+// slices of 32 or 48 channels, a shorter chain for more workgroups. 417 x 233:
+// 173 -> 98 us (large tiles there: 204); eight 128 x 128 images of a training
+// step: 1143 -> 990.
+struct ConvLarge {
+    static constexpr int R(int cout, int ng) { return cout <= 32 && ng > 1 ? 4 : 2; }
+    static constexpr int NT = 2, WR = 2, WC = 2;
+    static constexpr int CB(int cout) { return cout > 112 ? cout / 2 : cout; }
+};
+struct ConvSmall {
+    static constexpr int R(int, int) { return 1; }
+    static constexpr int NT = 1, WR = 4, WC = 1;
+    static constexpr int CB(int cout) { return cout % 48 == 0 ? 48 : (cout % 32 == 0 ? 32 : cout); }
+};
+struct ConvSmallPool : ConvSmall {   // a wave needs both rows of a 2 x 2 average
+    static constexpr int R(int, int) { return 2; }
+};
+constexpr int kConvThreads = 256;
+// Waves per SIMD that the LDS of one workgroup (halo tile + staged weights)
+// allows on a 160 KB CU, one wave per SIMD per workgroup, and that the
+// accumulators and the chunks in flight leave registers for: the register
+// budget is held to it.
+constexpr int conv_waves(int lds, int acc) {
+    const int w = 163840 / lds, v = acc <= 32 ? 3 : (acc <= 64 ? 2 : 1);
+    return w < 1 ? 1 : (w < v ? w : v);
 }
-template <int C0, int UP0, int C1, int COUT, int EPI>
-__global__ void __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(conv_waves(COUT)))) k_conv3x3(const __bf16* __restrict__ src0, const __bf16* __restrict__ src1,
-                                                     const __bf16* __restrict__ wgt, const float* __restrict__ bias,
-                                                     const __bf16* __restrict__ mask, void* __restrict__ out, uint32_t N,
-                                                     uint32_t H, uint32_t W) {
-    constexpr int CT = C0 + C1;
-    constexpr int K = 9 * CT;
-    constexpr int KPAD = (K + 31) / 32 * 32;
-    constexpr int MT = COUT / 16;
-    constexpr int NT = COUT <= 96 ? 4 : 2;
-    constexpr int TW = 16 * NT;
-    constexpr int TR = kConvRows + 2, TC = TW + 2;   // halo tile rows / columns
-    constexpr int NG = (CT + 31) / 32;       // channel groups of 32
-    static_assert(C0 % 8 == 0 && C1 % 8 == 0 && COUT % 16 == 0, "channel groups");
-    constexpr int TILE = TR * TC * 4;
-    constexpr int SPT = (TILE + kConvThreads - 1) / kConvThreads;  // staged 16-B chunks per thread
-    // [row][col][4 chunks of 8 channels], the chunks of pixel p stored in the
-    // order chunk ^ ((p >> 1) & 3), which spreads the fragment reads of
-    // neighbouring pixels over the banks
-    __shared__ bf16x8 tile[TILE];
-    // Up to 48 output channels, the group's weights are staged in LDS too
-    // ([tap][co] rows of 32 channels + 8 of padding, so the 16 rows a wave
-    // reads at once fall on distinct banks), loaded with the tile.
-    constexpr bool LDSW = COUT <= 96;
-    constexpr int WROW = 5;                  // 16-B chunks per (tap, co) row
-    constexpr int WCH = 9 * COUT * 4;        // weight chunks per group
-    constexpr int WPT = LDSW ? (WCH + kConvThreads - 1) / kConvThreads : 1;
-    __shared__ bf16x8 wl[LDSW ? 9 * COUT * WROW : 1];
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    const uint32_t r = lane & 15u, g = lane >> 4;
-    const uint32_t segs = (W + TW - 1) / TW, rblocks = (H + kConvRows - 1) / kConvRows;
-    const uint32_t blk = blockIdx.x;
-    const uint32_t seg = blk % segs, rest = blk / segs;
-    const uint32_t rb = rest % rblocks, n = rest / rblocks;
-    const int y0 = (int)(rb * kConvRows), x0 = (int)(seg * TW);
-    const uint32_t H0 = H / UP0, W0 = W / UP0;
-    const int y = y0 + (int)wv;
-
-    f32x4 acc[MT][NT];
+template <typename CFG, int C0, int C1, int COUT>
+struct ConvShape {
+    static constexpr int NG = (C0 + C1 + 31) / 32;           // groups of 32 channels
+    static constexpr int R = CFG::R(COUT, NG), NT = CFG::NT, WR = CFG::WR, WC = CFG::WC, CB = CFG::CB(COUT);
+    static constexpr int MT = CB / 16, ROWS = R * WR, COLS = 16 * NT * WC;
+    static constexpr int TR = ROWS + 2, TC = COLS + 2;       // halo tile
+    static constexpr int LDS = (TR * TC + 9 * CB) * 64, ACC = 4 * R * MT * NT;
+    static_assert(WR * WC * 64 == kConvThreads && COUT % CB == 0 && CB % 16 == 0, "workgroup shape");
+};
+// LC consecutive BF16 channels (LC a multiple of 4) as the widest aligned stores.
+template <int LC>
+__device__ inline void store_channels(__bf16* p, const __bf16* v) {
+    if constexpr (LC % 8 == 0) {
 #pragma unroll
-    for (int m = 0; m < MT; m++)
+        for (int j = 0; j < LC; j += 8) {
+            bf16x8 q;
 #pragma unroll
-        for (int t = 0; t < NT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // Halo tile of channels [32 cg, 32 cg + 32): every load of a thread is
-    // issued before any is stored, and before the barrier that waits for the
-    // previous group's MFMAs (the staging registers are dead during them).
-    bf16x8 stage[SPT];
-    bf16x8 wstage[WPT];
-    auto load_group = [&](int cg) {
-        if constexpr (LDSW) {
-#pragma unroll
-            for (int i = 0; i < WPT; i++) {
-                const int e = (int)threadIdx.x + i * kConvThreads;
-                const int j = e & 3, row = e >> 2;     // 8-channel chunk of row (tap, co)
-                const int co = row % COUT, tap = row / COUT;
-                const int c = cg * 32 + j * 8;
-                bf16x8 v = zero8();
-                if (e < WCH && c < CT) v = *(const bf16x8*)(wgt + (size_t)co * KPAD + tap * CT + c);
-                wstage[i] = v;
-            }
+            for (int i = 0; i < 8; i++) q[i] = v[j + i];
+            *(bf16x8*)(p + j) = q;
         }
+    } else {
 #pragma unroll
-        for (int i = 0; i < SPT; i++) {
-            const int e = (int)threadIdx.x + i * kConvThreads;
-            const int chunk = e & 3, pix = e >> 2;
-            const int ty = pix / TC, tx = pix - ty * TC;
-            const int sy = y0 - 1 + ty, sx = x0 - 1 + tx;
-            const int c = cg * 32 + chunk * 8;
-            bf16x8 v = zero8();
-            if (e < TILE && c < CT && sy >= 0 && sy < (int)H && sx >= 0 && sx < (int)W && n < N) {
-                const __bf16* p;
-                if (C1 == 0 || c < C0)
-                    p = src0 + (((size_t)n * H0 + (uint32_t)sy / UP0) * W0 + (uint32_t)sx / UP0) * C0 + c;
-                else
-                    p = src1 + (((size_t)n * H + (uint32_t)sy) * W + (uint32_t)sx) * C1 + (c - C0);
-                v = *(const bf16x8*)p;
-            }
-            stage[i] = v;
-        }
-    };
-    for (int cg = 0; cg < NG; cg++) {
-        load_group(cg);
-        __syncthreads();  // every wave is done reading the previous group
+        for (int j = 0; j < LC; j += 4) {
+            bf16x4 q;
 #pragma unroll
-        for (int i = 0; i < SPT; i++) {
-            const int e = (int)threadIdx.x + i * kConvThreads;
-            if (e < TILE) tile[(e & ~3) | ((e & 3) ^ ((e >> 3) & 3))] = stage[i];
-        }
-        if constexpr (LDSW) {
-#pragma unroll
-            for (int i = 0; i < WPT; i++) {
-                const int e = (int)threadIdx.x + i * kConvThreads;
-                if (e < WCH) wl[(e >> 2) * WROW + (e & 3)] = wstage[i];
-            }
-        }
-        __syncthreads();
-        const int c = cg * 32 + (int)g * 8;      // this lane's 8 channels
-        const bool cok = c < CT;
-#pragma unroll 3
-        for (int tap = 0; tap < 9; tap++) {
-            const int dy = tap / 3, dx = tap % 3;   // tile offsets (halo origin at -1)
-            bf16x8 b[NT];
-#pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const int pix = ((int)wv + dy) * TC + t * 16 + (int)r + dx;
-                b[t] = tile[pix * 4 + ((int)g ^ ((pix >> 1) & 3))];
-            }
-            const int k = tap * CT + c;
-#pragma unroll
-            for (int m = 0; m < MT; m++) {
-                bf16x8 a;
-                if constexpr (LDSW) a = wl[(tap * COUT + m * 16 + (int)r) * WROW + (int)g];
-                else a = cok ? *(const bf16x8*)(wgt + (size_t)(m * 16 + r) * KPAD + k) : zero8();
-#pragma unroll
-                for (int t = 0; t < NT; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[t], acc[m][t], 0, 0, 0);
-            }
+            for (int i = 0; i < 4; i++) q[i] = v[j + i];
+            *(bf16x4*)(p + j) = q;
         }
     }
-    if (y >= (int)H || n >= N) return;
+}
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// The value of the lane whose number differs in the last bit.
+__device__ inline bf16x2 lane_pair(bf16x2 v) {
+    return __builtin_bit_cast(bf16x2, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+}
+// a summed over lanes l and l + 32 in lanes 0-31, b likewise in lanes 32-63.
+__device__ inline float add_halves(float a, float b) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+    return __builtin_bit_cast(float, (uint32_t)s[0]) + __builtin_bit_cast(float, (uint32_t)s[1]);
+}
+// a summed over rows of 16 lanes 2k and 2k + 1 in row 2k, b likewise in row 2k + 1.
+__device__ inline float add_rows(float a, float b) {
+    const auto s = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+    return __builtin_bit_cast(float, (uint32_t)s[0]) + __builtin_bit_cast(float, (uint32_t)s[1]);
+}
+template <int C0, int UP0, int C1, int COUT, int EPI, typename CFG>
+__global__ void __launch_bounds__(kConvThreads)
+__attribute__((amdgpu_waves_per_eu(conv_waves(ConvShape<CFG, C0, C1, COUT>::LDS, ConvShape<CFG, C0, C1, COUT>::ACC))))
+k_conv3x3(const __bf16* __restrict__ src0, const __bf16* __restrict__ src1, const __bf16* __restrict__ wgt,
+          const float* __restrict__ bias, const __bf16* __restrict__ mask, void* __restrict__ out, uint32_t N, uint32_t H,
+          uint32_t W, ConvExtra ex) {
+    using SH = ConvShape<CFG, C0, C1, COUT>;
+    constexpr int CT = C0 + C1;
+    constexpr int KPAD = (9 * CT + 31) / 32 * 32;
+    constexpr int R = SH::R, NT = SH::NT, MT = SH::MT, CB = SH::CB, TR = SH::TR, TC = SH::TC;
+    constexpr bool SPLIT = EPI == EPI_SPLIT;
+    constexpr int G0 = (C0 + 31) / 32, NG = SPLIT ? G0 + (C1 + 31) / 32 : SH::NG;
+    static_assert(C0 % 8 == 0 && C1 % 8 == 0 && (UP0 == 1 || UP0 == 2), "channel groups");
+    // Halo tile: a thread stages one 8-channel chunk of one column in RPP rows
+    // at a time; columns past the 64th (of a tile 64 wide) are one more pass.
+    constexpr int ROWCH = TC * 4 > kConvThreads ? kConvThreads : TC * 4;
+    constexpr int RPP = kConvThreads / ROWCH, PASSES = (TR + RPP - 1) / RPP;
+    constexpr int EXTRA = TC * 4 - ROWCH;
+    static_assert(EXTRA * TR <= kConvThreads, "one more pass");
+    constexpr int SPT = PASSES + (EXTRA > 0 ? 1 : 0);
+    // Weights: CB rows of four chunks per tap.
+    constexpr int TAPCH = CB * 4, TPP = TAPCH > kConvThreads ? 1 : kConvThreads / TAPCH;
+    constexpr int PPT = (TAPCH + kConvThreads - 1) / kConvThreads;
+    constexpr int WPT = PPT * ((9 + TPP - 1) / TPP);
+    // [row][col][4 chunks of 8 channels], the chunks of pixel (row, col) stored
+    // in the order chunk ^ ((row + (col >> 1)) & 3), which spreads the fragment
+    // reads of neighbouring pixels over the banks
+    __shared__ bf16x8 tile[TR * TC * 4];
+    // [tap][row] weights; row m * 16 + 4 g + i holds output channel 4 MT g + 4 m + i,
+    // so that a lane's sums are 4 MT consecutive channels of its pixels; a row's
+    // four chunks are in the order chunk ^ ((row >> 1) & 3)
+    __shared__ bf16x8 wl[9 * CB * 4];
+    const int tid = (int)threadIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = tid & 15, g = (tid >> 4) & 3;
+    const uint32_t segs = (W + SH::COLS - 1) / SH::COLS, rblocks = (H + SH::ROWS - 1) / SH::ROWS;
+    const uint32_t tiles = N * rblocks * segs, step = gridDim.x;
+    const int cb0 = (int)blockIdx.y * CB;
+    const int wr = wv / SH::WC * R, wc = wv % SH::WC * NT * 16;   // the wave's part of the tile
+    struct Place { uint32_t n; int y0, x0; };
+    auto place = [&](uint32_t tl) {
+        const uint32_t rest = __builtin_amdgcn_readfirstlane(tl / segs), n = __builtin_amdgcn_readfirstlane(rest / rblocks);
+        return Place{n, (int)((rest - n * rblocks) * SH::ROWS), (int)((tl - rest * segs) * SH::COLS)};
+    };
+
+    const int prow = RPP == 1 ? 0 : tid / ROWCH, pcol = (tid - prow * ROWCH) >> 2, pchunk = tid & 3;
+    static_assert(ROWCH % 4 == 0, "a thread's chunk is tid & 3");
+    const int wtap = TPP == 1 ? 0 : tid / TAPCH, wrow0 = (tid - wtap * TAPCH) >> 2;
+    bf16x8 stage[SPT], wstage[WPT];
+    // Channel group cg of tile tl: every load of a thread is issued before any
+    // is stored. Lanes with nothing to load ask for an offset past the end of
+    // the buffer descriptor, which returns zeros.
+    constexpr uint32_t kEnd = 0x7FFFFFFFu, kNone = 0x80000000u, kRaw = 0x00020000u;
+    // `kc` is the group's first channel in `src` (negative if the other source has it).
+    auto load_tile = [&](const Place& p, const __bf16* src, int C, int up, int kc) {
+        const uint32_t HS = H >> up, WS = W >> up;
+        const bool chunk_ok = kc + pchunk * 8 < C;
+        const int sx = p.x0 - 1 + pcol;
+        const bool col_ok = chunk_ok && (uint32_t)sx < W;
+        if constexpr (RPP == 1) {
+            // one row per pass: its address is the wave's
+            const uint32_t off = col_ok && pcol * 4 < ROWCH ? (uint32_t)(((pcol + up) >> up) * C + pchunk * 8) * 2u : kNone;
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const uint32_t x = (uint32_t)x0 + t * 16 + r;
-        if (x >= W) continue;
-        const size_t pix = ((size_t)n * H + (uint32_t)y) * W + x;
-#pragma unroll
-        for (int m = 0; m < MT; m++) {
-            const int co = m * 16 + (int)g * 4;
-            f32x4 v = acc[m][t];
-            if (EPI == EPI_F32) {
-                *(f32x4*)((float*)out + pix * COUT + co) = v;
-                continue;
+            for (int i = 0; i < PASSES; i++) {
+                const int sy = p.y0 - 1 + i;
+                const __bf16* base = src + (((int64_t)p.n * HS + (sy >> up)) * WS + (p.x0 >> up) - 1) * C + kc;
+                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (uint32_t)sy < H ? kEnd : 0u, kRaw);
+                stage[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
             }
-            if (EPI == EPI_BIAS_RELU) {
+        } else {
+            // offsets within one image, which is small here
+            const __bf16* base = src + (int64_t)p.n * HS * WS * C + kc;
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, kEnd, kRaw);
 #pragma unroll
-                for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i] + bias[co + i], 0.0f);
+            for (int i = 0; i < PASSES; i++) {
+                const int ty = i * RPP + prow, sy = p.y0 - 1 + ty;
+                const bool ok = col_ok && prow < RPP && ty < TR && (uint32_t)sy < H;
+                const uint32_t off = ok ? (uint32_t)(((sy >> up) * (int)WS + (sx >> up)) * C + pchunk * 8) * 2u : kNone;
+                stage[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+            }
+        }
+        if constexpr (EXTRA > 0) {
+            const int ty = tid / EXTRA, ex_x = p.x0 - 1 + ROWCH / 4 + ((tid % EXTRA) >> 2), sy = p.y0 - 1 + ty;
+            bf16x8 v = zero8();
+            if (ty < TR && chunk_ok && (uint32_t)sy < H && (uint32_t)ex_x < W)
+                v = *(const bf16x8*)(src + (((size_t)p.n * HS + (uint32_t)(sy >> up)) * WS + (uint32_t)(ex_x >> up)) * C + (kc + pchunk * 8));
+            stage[PASSES] = v;
+        }
+    };
+    auto load_group = [&](uint32_t tl, int cg, bool weights) {
+        if (weights) {
+            const int c = SPLIT && cg >= G0 ? C0 + (cg - G0) * 32 : cg * 32, end = SPLIT && cg < G0 ? C0 : CT;
+            const __bf16* base = wgt + (size_t)cb0 * KPAD + c;
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, kEnd, kRaw);
+#pragma unroll
+            for (int i = 0; i < WPT; i++) {
+                const int row = wrow0 + (i % PPT) * (kConvThreads / 4), tap0 = i / PPT * TPP;
+                const bool ok = c + pchunk * 8 < end && row < CB && wtap < TPP && tap0 + wtap < 9;
+                const uint32_t off = ok ? (uint32_t)(row * KPAD + wtap * CT + pchunk * 8) * 2u : kNone;
+                wstage[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, off, tap0 * CT * 2, 0));
+            }
+        }
+        const Place p = place(tl);
+        if constexpr (SPLIT) {
+            load_tile(p, cg < G0 ? src0 : src1, cg < G0 ? C0 : C1, cg < G0 ? UP0 - 1 : 0, (cg < G0 ? cg : cg - G0) * 32);
+        } else if constexpr (C1 != 0 && C0 % 32 != 0) {   // a group may have chunks of both sources
+            if (cg * 32 + pchunk * 8 < C0) load_tile(p, src0, C0, UP0 - 1, cg * 32);
+            else load_tile(p, src1, C1, 0, cg * 32 - C0);
+        } else {
+            const bool first = C1 == 0 || cg * 32 < C0;
+            load_tile(p, first ? src0 : src1, first ? C0 : C1, first ? UP0 - 1 : 0, first ? cg * 32 : cg * 32 - C0);
+        }
+    };
+    auto slot = [](int ty, int tx, int chunk) { return (ty * TC + tx) * 4 + (chunk ^ ((ty + (tx >> 1)) & 3)); };
+    auto store_group = [&](bool weights) {
+#pragma unroll
+        for (int i = 0; i < PASSES; i++) {
+            const int ty = i * RPP + prow;
+            if (RPP == 1 ? pcol * 4 < ROWCH : prow < RPP && ty < TR) tile[slot(ty, pcol, pchunk)] = stage[i];
+        }
+        if constexpr (EXTRA > 0) {
+            const int ty = tid / EXTRA;
+            if (ty < TR) tile[slot(ty, ROWCH / 4 + ((tid % EXTRA) >> 2), pchunk)] = stage[PASSES];
+        }
+        if (weights) {
+#pragma unroll
+            for (int i = 0; i < WPT; i++) {
+                const int co = wrow0 + (i % PPT) * (kConvThreads / 4), tap = i / PPT * TPP + wtap;
+                const int row = (co % (4 * MT)) / 4 * 16 + co / (4 * MT) * 4 + (co & 3);
+                if (co < CB && wtap < TPP && tap < 9)
+                    wl[(tap * CB + row) * 4 + (pchunk ^ ((row >> 1) & 3))] = wstage[i];
+            }
+        }
+    };
+    // The next group's (or tile's) loads are in flight during a group's MFMAs
+    // and a tile's stores; the weights of a single group stay in LDS.
+    bool weights = true;
+    uint32_t tl = blockIdx.x;
+    if (tl < tiles) load_group(tl, 0, true);
+    for (; tl < tiles; tl += step) {
+        f32x4 acc[R][MT][NT];
+#pragma unroll
+        for (int o = 0; o < R; o++)
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) acc[o][m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int cg = 0; cg < NG; cg++) {
+            __syncthreads();  // every wave is done reading the previous group
+            store_group(weights);
+            __syncthreads();
+            weights = NG > 1;
+            if (cg + 1 < NG) load_group(tl, cg + 1, true);
+            else if (tl + step < tiles) load_group(tl + step, 0, weights);
+            if constexpr (SPLIT) {
+#pragma unroll
+                for (int dx = 0; dx < 3; dx++) {
+                    bf16x8 a[3][MT];
+#pragma unroll
+                    for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+                        for (int m = 0; m < MT; m++)
+                            a[dy][m] = wl[((dy * 3 + dx) * CB + m * 16 + r) * 4 + (g ^ ((r >> 1) & 3))];
+                    const int col = wc + r + dx;             // tile column (of pixel t = 0)
+#pragma unroll
+                    for (int ir = 0; ir < R + 2; ir++) {
+                        const bf16x8* row = tile + ((wr + ir) * TC + col) * 4 + (g ^ ((wr + ir + (col >> 1)) & 3));
+#pragma unroll
+                        for (int t = 0; t < NT; t++) {
+                            const bf16x8 b = row[t * 64];
+#pragma unroll
+                            for (int dy = 0; dy < 3; dy++) {
+                                const int o = ir - dy;
+                                if (o < 0 || o >= R) continue;
+#pragma unroll
+                                for (int m = 0; m < MT; m++)
+                                    acc[o][m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[dy][m], b, acc[o][m][t], 0, 0, 0);
+                            }
+                        }
+                    }
+                }
             } else {
-                const bf16x4 mk = *(const bf16x4*)(mask + pix * COUT + co);
 #pragma unroll
-                for (int i = 0; i < 4; i++) v[i] = (float)mk[i] > 0.0f ? v[i] : 0.0f;
+                for (int dy = 0; dy < 3; dy++) {
+                    // 32 channels leave 168 registers to three waves: loads of a
+                    // later row moved up here would spill where these epilogues
+                    // or two sources add to them
+                    if constexpr (CB == 32 && (EPI == EPI_POOL || EPI == EPI_HEAD || C1 != 0))
+                        if (dy > 0) __builtin_amdgcn_sched_barrier(0);
+                    bf16x8 a[3][MT];
+#pragma unroll
+                    for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+                        for (int m = 0; m < MT; m++)
+                            a[dx][m] = wl[((dy * 3 + dx) * CB + m * 16 + r) * 4 + (g ^ ((r >> 1) & 3))];
+#pragma unroll
+                    for (int o = 0; o < R; o++)
+#pragma unroll
+                        for (int dx = 0; dx < 3; dx++) {
+                            const int col = wc + r + dx;     // tile column (of pixel t = 0)
+                            const bf16x8* row = tile + ((wr + o + dy) * TC + col) * 4 + (g ^ ((wr + o + dy + (col >> 1)) & 3));
+#pragma unroll
+                            for (int t = 0; t < NT; t++) {
+                                const bf16x8 b = row[t * 64];
+#pragma unroll
+                                for (int m = 0; m < MT; m++)
+                                    acc[o][m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[dx][m], b, acc[o][m][t], 0, 0, 0);
+                            }
+                        }
+                }
             }
-            bf16x4 o;
+        }
+
+        const Place p = place(tl);
+        constexpr int LC = 4 * MT;                        // channels of this lane: c0 .. c0 + LC - 1
+        const int c0 = cb0 + LC * g;
+        // pixel (o, t) of this lane: row y(o), column x(t), at `px` channels of the row's `wide`
+        auto y = [&](int o) { return (uint32_t)(p.y0 + wr + o); };
+        auto x = [&](int t) { return (uint32_t)(p.x0 + wc + t * 16 + r); };
+        auto first_pixel = [&](int o, int t) { return ((size_t)p.n * H + y(o)) * W + (uint32_t)(p.x0 + wc + t * 16); };
+        const uint32_t mine = (uint32_t)(r * COUT + c0);
+        if constexpr (EPI == EPI_F32 || EPI == EPI_MASK) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) o[i] = (__bf16)v[i];
-            *(bf16x4*)((__bf16*)out + pix * COUT + co) = o;
+            for (int o = 0; o < R; o++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    if (y(o) >= H || x(t) >= W) continue;
+                    const size_t at = first_pixel(o, t) * COUT;
+#pragma unroll
+                    for (int m = 0; m < MT; m++) {
+                        const f32x4 v = acc[o][m][t];
+                        if constexpr (EPI == EPI_F32) {
+                            *(f32x4*)((float*)out + at + (mine + 4 * m)) = v;
+                        } else {
+                            const bf16x4 mk = *(const bf16x4*)(mask + at + (mine + 4 * m));
+                            bf16x4 q;
+#pragma unroll
+                            for (int i = 0; i < 4; i++) q[i] = (__bf16)((float)mk[i] > 0.0f ? v[i] : 0.0f);
+                            *(bf16x4*)((__bf16*)out + at + (mine + 4 * m)) = q;
+                        }
+                    }
+                }
+        } else {
+            f32x4 bv[MT];
+#pragma unroll
+            for (int m = 0; m < MT; m++) bv[m] = *(const f32x4*)(bias + c0 + 4 * m);
+            __bf16 q[R][NT][LC];
+#pragma unroll
+            for (int o = 0; o < R; o++)
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int j = 0; j < LC; j++) q[o][t][j] = (__bf16)fmaxf(acc[o][j / 4][t][j & 3] + bv[j / 4][j & 3], 0.0f);
+            if constexpr (EPI != EPI_HEAD) {
+#pragma unroll
+                for (int o = 0; o < R; o++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++) {
+                        if (y(o) >= H || x(t) >= W) continue;
+                        store_channels<LC>((__bf16*)out + first_pixel(o, t) * COUT + mine, q[o][t]);
+                    }
+            }
+            if constexpr (EPI == EPI_POOL) {
+                // 2 x 2 averages of the stored values; the right pixel is the
+                // next lane's (x0, wc and 16 t are even, as are H and W)
+                static_assert(R % 2 == 0, "a wave holds whole row pairs");
+#pragma unroll
+                for (int o = 0; o < R; o += 2)
+#pragma unroll
+                    for (int t = 0; t < NT; t++) {
+                        __bf16 a[LC];
+#pragma unroll
+                        for (int j = 0; j < LC; j += 2) {
+                            const bf16x2 u = {q[o][t][j], q[o][t][j + 1]}, l = {q[o + 1][t][j], q[o + 1][t][j + 1]};
+                            const bf16x2 u1 = lane_pair(u), l1 = lane_pair(l);
+#pragma unroll
+                            for (int i = 0; i < 2; i++)
+                                a[j + i] = (__bf16)(((((float)u[i] + (float)u1[i]) + (float)l[i]) + (float)l1[i]) * 0.25f);
+                        }
+                        if (y(o) >= H || x(t) >= W || (r & 1) != 0) continue;
+                        const size_t at = ((size_t)p.n * (H / 2) + y(o) / 2) * (W / 2) + (uint32_t)(p.x0 + wc + t * 16) / 2;
+                        store_channels<LC>(ex.pool + at * COUT + (uint32_t)(r / 2 * COUT + c0), a);
+                    }
+            }
+            if constexpr (EPI == EPI_HEAD) {
+                // out = W_head a + b + residual: partial sums over the lane's
+                // channels, added over the four lanes of a pixel such that
+                // each of them has the sums of a quarter of the wave's pixels
+                constexpr int P = R * NT;
+                static_assert(CB == COUT && (P == 1 || P == 4), "every channel of a pixel in one wave");
+                float v[3];
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    float s[P];
+#pragma unroll
+                    for (int q0 = 0; q0 < P; q0++) s[q0] = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < LC; j += 4) {
+                        const bf16x4 wk = *(const bf16x4*)(ex.wh + k * COUT + c0 + j);
+#pragma unroll
+                        for (int i = 0; i < 4; i++)
+#pragma unroll
+                            for (int q0 = 0; q0 < P; q0++) s[q0] = fmaf((float)wk[i], (float)q[q0 / NT][q0 % NT][j + i], s[q0]);
+                    }
+                    if constexpr (P == 4) v[k] = add_rows(add_halves(s[0], s[1]), add_halves(s[2], s[3]));
+                    else v[k] = add_rows(add_halves(s[0], s[0]), add_halves(s[0], s[0]));
+                }
+                // add_halves leaves its first argument's sums in lanes 0-31, its
+                // second's in 32-63; add_rows its first's in even rows of 16
+                const int q0 = P == 4 ? (g >> 1) + 2 * (g & 1) : 0, o = q0 / NT, t = q0 % NT;
+                const uint32_t yy = y(o), xx = x(t);
+                if ((P > 1 || g == 0) && yy < H && xx < W) {
+                    const size_t pix = ((size_t)p.n * H + yy) * W + xx;
+                    const float4 rs = ex.resid[pix];
+                    const float4 res = make_float4(v[0] + ex.bh[0] + rs.x, v[1] + ex.bh[1] + rs.y, v[2] + ex.bh[2] + rs.z, 0.0f);
+                    if (ex.out) ex.out[pix] = res;
+                    if (ex.surface && p.n == 0 && xx < ex.w && yy < ex.h)
+                        ex.surface[(size_t)yy * ex.w + xx] = make_float4(fmaxf(expm1f(res.x), 0.0f), fmaxf(expm1f(res.y), 0.0f),
+                                                                         fmaxf(expm1f(res.z), 0.0f), 1.0f);
+                }
+            }
         }
     }
 }
@@ -421,31 +698,6 @@ __global__ void __launch_bounds__(256) k_reduce_grads(GradSlices t) {
 // ---------------------------------------------------------------------------
 // Pooling and the gradients of upsampling / pooling
 // ---------------------------------------------------------------------------
-// 2x2 average; one thread = one output pixel x 8 channels.
-__global__ void k_pool2(const __bf16* __restrict__ in, __bf16* __restrict__ out, uint32_t N, uint32_t H, uint32_t W,
-                        uint32_t C) {
-    const uint32_t Ho = H / 2, Wo = W / 2, G = C / 8;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)N * Ho * Wo * G) return;
-    const uint32_t gi = (uint32_t)(i % G);
-    size_t q = i / G;
-    const uint32_t xo = (uint32_t)(q % Wo);
-    q /= Wo;
-    const uint32_t yo = (uint32_t)(q % Ho), n = (uint32_t)(q / Ho);
-    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int d = 0; d < 4; d++) {
-        const size_t pix = ((size_t)n * H + 2 * yo + (d >> 1)) * W + 2 * xo + (d & 1);
-        const bf16x8 v = *(const bf16x8*)(in + pix * C + gi * 8);
-#pragma unroll
-        for (int e = 0; e < 8; e++) s[e] += (float)v[e];
-    }
-    bf16x8 o;
-#pragma unroll
-    for (int e = 0; e < 8; e++) o[e] = (__bf16)(s[e] * 0.25f);
-    *(bf16x8*)(out + i * 8) = o;
-}
-
 // Gradient of "upsample then concatenate" for the upsampled part: the sum of
 // the four children (channels [0, C0) of the FP32 input gradient, CT wide),
 // times the ReLU mask of the low-resolution activation -> BF16.
@@ -526,15 +778,16 @@ __device__ inline void octahedral(float x, float y, float z, float& ox, float& o
 // log radiance for the head's residual. Source: either raw records
 // (12 floats per pixel: radiance, albedo, depth code, normal, M2, samples)
 // or a surface (radiance plane + two feature planes, `held` samples).
-// Pixels of the padded network image outside (h, w) are zero.
+// Pixels of the padded network image outside (h, w) are zero. A wave takes 64
+// pixels of a row (the row is the wave's, so no lane divides).
 __global__ void k_pack(const float* __restrict__ raw, const float4* __restrict__ rad, const float4* __restrict__ aux,
                        uint32_t held, uint32_t N, uint32_t h, uint32_t w, uint32_t Hp, uint32_t Wp,
                        __bf16* __restrict__ xin, float4* __restrict__ resid) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)N * Hp * Wp) return;
-    const uint32_t x = (uint32_t)(i % Wp);
-    const size_t q = i / Wp;
-    const uint32_t y = (uint32_t)(q % Hp), n = (uint32_t)(q / Hp);
+    const uint32_t segs = (Wp + 63) / 64, rb = blockIdx.x / segs;
+    const uint32_t row = __builtin_amdgcn_readfirstlane(rb * 4 + threadIdx.x / 64), n = row / Hp, y = row - n * Hp;
+    const uint32_t x = (blockIdx.x - rb * segs) * 64 + threadIdx.x % 64;
+    if (n >= N || x >= Wp) return;
+    const size_t i = (size_t)row * Wp + x;
     float f[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const bool valid = x < w && y < h;
     if (valid) {
@@ -588,8 +841,7 @@ __global__ void k_pack(const float* __restrict__ raw, const float4* __restrict__
 // 1x1 head: out = W_head (3 x 32) . act + b + residual (FP32). Optionally also
 // writes the denoised radiance max(expm1(out), 0) into an RGBA32F surface.
 __global__ void k_head(const __bf16* __restrict__ act, const __bf16* __restrict__ wh, const float* __restrict__ bh,
-                       const float4* __restrict__ resid, float4* __restrict__ out, uint32_t N, uint32_t Hp, uint32_t Wp,
-                       float4* __restrict__ surface, uint32_t h, uint32_t w) {
+                       const float4* __restrict__ resid, float4* __restrict__ out, uint32_t N, uint32_t Hp, uint32_t Wp) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)N * Hp * Wp) return;
     float o[3];
@@ -606,16 +858,7 @@ __global__ void k_head(const __bf16* __restrict__ act, const __bf16* __restrict_
         }
     }
     const float4 rs = resid[i];
-    const float4 res = make_float4(o[0] + bh[0] + rs.x, o[1] + bh[1] + rs.y, o[2] + bh[2] + rs.z, 0.0f);
-    out[i] = res;
-    if (surface) {
-        const uint32_t x = (uint32_t)(i % Wp);
-        const size_t q = i / Wp;
-        const uint32_t y = (uint32_t)(q % Hp), n = (uint32_t)(q / Hp);
-        if (n == 0 && x < w && y < h)
-            surface[(size_t)y * w + x] =
-                make_float4(fmaxf(expm1f(res.x), 0.0f), fmaxf(expm1f(res.y), 0.0f), fmaxf(expm1f(res.z), 0.0f), 1.0f);
-    }
+    out[i] = make_float4(o[0] + bh[0] + rs.x, o[1] + bh[1] + rs.y, o[2] + bh[2] + rs.z, 0.0f);
 }
 
 // Loss over the valid pixels (0 gradient on padding); the sum goes to *loss.
@@ -769,12 +1012,31 @@ __global__ void k_zero_f32(float* __restrict__ p, size_t n) {
 // ---------------------------------------------------------------------------
 static inline uint32_t cdiv(size_t a, uint32_t b) { return (uint32_t)((a + b - 1) / b); }
 
+// Large tiles from one workgroup per CU on. The whole network at 417 x 233 and
+// 1280 x 720, training step of eight 128 x 128: from 128 workgroups 94, 333 us
+// and 1005; from 256 97, 339 and 990; from 512 101, 337 and 990; from 1024 102,
+// 361 and 1006 (800 x 600: 222, 215, 214 and 226).
+constexpr uint32_t kConvFill = 256;
+template <typename SHAPE>
+static uint32_t conv_tiles(uint32_t N, uint32_t H, uint32_t W) {
+    return N * cdiv(H, SHAPE::ROWS) * cdiv(W, SHAPE::COLS);
+}
 template <int C0, int UP0, int C1, int COUT, int EPI>
 static void conv(hipStream_t st, const __bf16* s0, const __bf16* s1, const __bf16* w, const float* b, const __bf16* mask,
-                 void* out, uint32_t N, uint32_t H, uint32_t W) {
-    constexpr int NT = COUT <= 96 ? 4 : 2;
-    const size_t blocks = (size_t)N * ((H + kConvRows - 1) / kConvRows) * ((W + 16 * NT - 1) / (16 * NT));
-    k_conv3x3<C0, UP0, C1, COUT, EPI><<<(uint32_t)blocks, kConvThreads, 0, st>>>(s0, s1, w, b, mask, out, N, H, W);
+                 void* out, uint32_t N, uint32_t H, uint32_t W, const ConvExtra& ex = ConvExtra{}) {
+    using LG = ConvLarge;
+    using SM = std::conditional_t<EPI == EPI_POOL, ConvSmallPool, ConvSmall>;
+    using LS = ConvShape<LG, C0, C1, COUT>;
+    using SS = ConvShape<SM, C0, C1, COUT>;
+    constexpr uint32_t ls = COUT / LS::CB, ss = COUT / SS::CB;
+    const uint32_t large = conv_tiles<LS>(N, H, W), small = conv_tiles<SS>(N, H, W);
+    if (large * ls >= kConvFill) {
+        constexpr uint32_t resident = 256 * conv_waves(LS::LDS, LS::ACC);
+        k_conv3x3<C0, UP0, C1, COUT, EPI, LG><<<dim3(std::min(large, resident / ls), ls), kConvThreads, 0, st>>>(
+            s0, s1, w, b, mask, out, N, H, W, ex);
+    } else {
+        k_conv3x3<C0, UP0, C1, COUT, EPI, SM><<<dim3(small, ss), kConvThreads, 0, st>>>(s0, s1, w, b, mask, out, N, H, W, ex);
+    }
 }
 
 // Layer table (matches oracle/unet.py LAYERS): c0, up0, c1, cout, level.
@@ -983,39 +1245,53 @@ void Net::release() {
 
 hipError_t Net::pack(hipStream_t st, const float* raw, const float4* rad, const float4* aux, uint32_t held, uint32_t h,
                      uint32_t w) {
-    k_pack<<<cdiv((size_t)n * H * W, 256), 256, 0, st>>>(raw, rad, aux, held, n, h, w, H, W, xin, (float4*)resid);
+    k_pack<<<cdiv(W, 64) * cdiv((size_t)n * H, 4), 256, 0, st>>>(raw, rad, aux, held, n, h, w, H, W, xin, (float4*)resid);
     return hipGetLastError();
 }
 
-hipError_t Net::forward(hipStream_t st, float4* surface, uint32_t h, uint32_t w) {
+// `training` keeps the last activation (the backward pass reads it); else the
+// head is part of the last convolution, which writes the surface when there is
+// one and the network output when there is not.
+hipError_t Net::forward(hipStream_t st, float4* surface, uint32_t h, uint32_t w, bool training) {
     const float* b[kDnLayers];
     for (int l = 0; l < kDnLayers; l++) b[l] = master + w_off[l] + (size_t)kLayers[l].cout * 9 * kLayers[l].cin_real;
     const uint32_t N = n;
     auto Hl = [&](int lv) { return H >> lv; };
     auto Wl = [&](int lv) { return W >> lv; };
-    auto pool2 = [&](int k, int l, int lv) {
-        const uint32_t C = kLayers[l].cout;
-        k_pool2<<<cdiv((size_t)N * Hl(lv + 1) * Wl(lv + 1) * (C / 8), 256), 256, 0, st>>>(act[l], pool[k], N, Hl(lv), Wl(lv), C);
+    auto pooled = [&](int k) {
+        ConvExtra ex{};
+        ex.pool = pool[k];
+        return ex;
     };
     conv<16, 1, 0, 32, EPI_BIAS_RELU>(st, xin, nullptr, wf[0], b[0], nullptr, act[0], N, Hl(0), Wl(0));
-    conv<32, 1, 0, 32, EPI_BIAS_RELU>(st, act[0], nullptr, wf[1], b[1], nullptr, act[1], N, Hl(0), Wl(0));
-    pool2(0, 1, 0);
+    conv<32, 1, 0, 32, EPI_POOL>(st, act[0], nullptr, wf[1], b[1], nullptr, act[1], N, Hl(0), Wl(0), pooled(0));
     conv<32, 1, 0, 48, EPI_BIAS_RELU>(st, pool[0], nullptr, wf[2], b[2], nullptr, act[2], N, Hl(1), Wl(1));
-    conv<48, 1, 0, 48, EPI_BIAS_RELU>(st, act[2], nullptr, wf[3], b[3], nullptr, act[3], N, Hl(1), Wl(1));
-    pool2(1, 3, 1);
+    conv<48, 1, 0, 48, EPI_POOL>(st, act[2], nullptr, wf[3], b[3], nullptr, act[3], N, Hl(1), Wl(1), pooled(1));
     conv<48, 1, 0, 64, EPI_BIAS_RELU>(st, pool[1], nullptr, wf[4], b[4], nullptr, act[4], N, Hl(2), Wl(2));
-    conv<64, 1, 0, 64, EPI_BIAS_RELU>(st, act[4], nullptr, wf[5], b[5], nullptr, act[5], N, Hl(2), Wl(2));
-    pool2(2, 5, 2);
+    conv<64, 1, 0, 64, EPI_POOL>(st, act[4], nullptr, wf[5], b[5], nullptr, act[5], N, Hl(2), Wl(2), pooled(2));
     conv<64, 1, 0, 96, EPI_BIAS_RELU>(st, pool[2], nullptr, wf[6], b[6], nullptr, act[6], N, Hl(3), Wl(3));
     conv<96, 1, 0, 96, EPI_BIAS_RELU>(st, act[6], nullptr, wf[7], b[7], nullptr, act[7], N, Hl(3), Wl(3));
     conv<96, 2, 64, 64, EPI_BIAS_RELU>(st, act[7], act[5], wf[8], b[8], nullptr, act[8], N, Hl(2), Wl(2));
     conv<64, 1, 0, 64, EPI_BIAS_RELU>(st, act[8], nullptr, wf[9], b[9], nullptr, act[9], N, Hl(2), Wl(2));
     conv<64, 2, 48, 48, EPI_BIAS_RELU>(st, act[9], act[3], wf[10], b[10], nullptr, act[10], N, Hl(1), Wl(1));
     conv<48, 1, 0, 48, EPI_BIAS_RELU>(st, act[10], nullptr, wf[11], b[11], nullptr, act[11], N, Hl(1), Wl(1));
-    conv<48, 2, 32, 32, EPI_BIAS_RELU>(st, act[11], act[1], wf[12], b[12], nullptr, act[12], N, Hl(0), Wl(0));
-    conv<32, 1, 0, 32, EPI_BIAS_RELU>(st, act[12], nullptr, wf[13], b[13], nullptr, act[13], N, Hl(0), Wl(0));
-    k_head<<<cdiv((size_t)N * H * W, 256), 256, 0, st>>>(act[13], whead, master + w_off[kDnLayers] + 96, (const float4*)resid,
-                                                         (float4*)out, N, H, W, surface, h, w);
+    if (training) conv<48, 2, 32, 32, EPI_BIAS_RELU>(st, act[11], act[1], wf[12], b[12], nullptr, act[12], N, Hl(0), Wl(0));
+    else conv<48, 2, 32, 32, EPI_SPLIT>(st, act[11], act[1], wf[12], b[12], nullptr, act[12], N, Hl(0), Wl(0));
+    const float* bh = master + w_off[kDnLayers] + 96;
+    if (training) {
+        conv<32, 1, 0, 32, EPI_BIAS_RELU>(st, act[12], nullptr, wf[13], b[13], nullptr, act[13], N, Hl(0), Wl(0));
+        k_head<<<cdiv((size_t)N * H * W, 256), 256, 0, st>>>(act[13], whead, bh, (const float4*)resid, (float4*)out, N, H, W);
+        return hipGetLastError();
+    }
+    ConvExtra ex{};
+    ex.wh = whead;
+    ex.bh = bh;
+    ex.resid = (const float4*)resid;
+    ex.out = surface ? nullptr : (float4*)out;
+    ex.surface = surface;
+    ex.h = h;
+    ex.w = w;
+    conv<32, 1, 0, 32, EPI_HEAD>(st, act[12], nullptr, wf[13], b[13], nullptr, nullptr, N, Hl(0), Wl(0), ex);
     return hipGetLastError();
 }
 

@@ -144,6 +144,27 @@ def test_gradients_at_strip_edges(dn, n, h, w):
             assert rel(a, b) <= 3e-2 and cos >= 0.999, (name, what, rel(a, b), cos)
 
 
+@pytest.mark.parametrize("n,h,w", [(3, 168, 72), (3, 176, 72), (1, 64, 1024), (2, 19, 135), (1, 8200, 8)])
+def test_convolution_tiles(dn, n, h, w):
+    """Convolutions at the edges of their two tile shapes: full-resolution
+    layers with 252 and 264 large tiles (256 is the least that takes them), 256
+    whole ones, ragged columns and rows on the small tiles, and an image whose
+    every level takes large tiles, more than are resident at once. Output as in
+    test_forward_padding, gradients as above, with the same bars."""
+    rng = np.random.default_rng(h + w)
+    params = perturbed_params(8)
+    dn.set_params(unet.flatten(params).astype(np.float32))
+    feats = random_feats(rng, n, h, w)
+    padded = np.zeros((n, (h + 7) // 8 * 8, (w + 7) // 8 * 8, unet.N_FEAT), np.float32)
+    padded[:, :h, :w] = feats
+    x = unet.pack_inputs(padded)
+    x[:, h:], x[:, :, w:] = 0.0, 0.0
+    ref, _ = unet.forward(params, x, emulate_bf16=True)
+    got = dn.forward(feats)
+    assert rel(got, ref[:, :h, :w]) <= 5e-3
+    test_gradients_at_strip_edges(dn, n, h, w)
+
+
 def test_training_lowers_loss(gpu_ctx):
     """A fixed batch of noisy constant patches: 60 Adam steps cut the loss."""
     from helios_amd.denoise import Denoiser
