@@ -548,28 +548,21 @@ struct QueueCursor {
     __device__ inline QueueCursor(const uint32_t* count_, uint32_t* head_, uint32_t seg_, uint32_t refill_)
         : count(count_), head(head_), seg(seg_), refill(refill_), shard(wave_shard()), tried(0u), drained(false) {}
     // Queue entry for this lane (kNoEntry: none). Called by the whole wave in
-    // converged control flow. With QUAD the four lanes of a quad are idle
-    // together and get one entry; `refill` counts lanes either way.
-    template <bool QUAD = false>
+    // converged control flow.
     __device__ inline uint32_t next(bool idle_lane) {
         if (drained) return kNoEntry;
-        unsigned long long idle = __ballot(idle_lane);
-        uint32_t nidle = (uint32_t)__popcll(idle);
+        const unsigned long long idle = __ballot(idle_lane);
+        const uint32_t nidle = (uint32_t)__popcll(idle);
         if (nidle < refill && nidle != 64u) return kNoEntry;
-        if (QUAD) {
-            idle &= 0x1111111111111111ull;   // one lane per quad
-            nidle >>= 2;
-        }
         // idle lanes below this one (mbcnt: no lane mask or lane index kept
         // in registers); the lowest idle lane (rank 0) claims for the wave
-        uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
-        if (QUAD && (lane_id() & 3u) != 0u) rank--;   // the quad's own bit
+        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
         uint32_t got = kNoEntry, done = 0u;
         while (done < nidle) {
             const uint32_t want = nidle - done;
             const uint32_t n = count[shard * kCtrStride];
             uint32_t base = 0;
-            if (idle_lane && rank == 0u && (!QUAD || (lane_id() & 3u) == 0u)) base = atomicAdd(head + shard * kCtrStride, want);
+            if (idle_lane && rank == 0u) base = atomicAdd(head + shard * kCtrStride, want);
             base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)__builtin_ctzll(idle));
             const uint32_t avail = base < n ? min(n - base, want) : 0u;
             if (idle_lane && rank >= done && rank < done + avail) got = shard * seg + base + (rank - done);
@@ -1043,35 +1036,6 @@ __global__ void __launch_bounds__(kAccBlock) k_accumulate(const ViewGPU* __restr
     }
 }
 
-// One way to trace a ray to its end with the lanes a path has: one lane
-// (any node layout) or a quad (BVH4). trace() leaves the hit in every lane of
-// the path.
-template <int W, bool QUAD>
-struct PathTracer {
-    LaneStack stk;
-    __device__ inline PathTracer(uint32_t* stack, uint32_t* spill, uint32_t bs)
-        : stk{to_lds(&stack[threadIdx.x]), bs, to_global(spill + blockIdx.x * bs + threadIdx.x), gridDim.x * bs} {}
-    template <bool ANY>
-    __device__ inline bool trace(const SceneGPU& S, f3 o, f3 d, float tmin, float tmax, uint32_t rflags, HitRec& h) const {
-        return trace_ray<W, ANY>(S, o, d, tmin, tmax, rflags, h, stk);
-    }
-};
-template <int W>
-struct PathTracer<W, true> {
-    QuadStack qs;
-    __device__ inline PathTracer(uint32_t* stack, uint32_t* spill, uint32_t bs) : qs(quad_stack(stack, spill, bs, gridDim.x)) {}
-    template <bool ANY>
-    __device__ inline bool trace(const SceneGPU& S, f3 o, f3 d, float tmin, float tmax, uint32_t rflags, HitRec& h) const {
-        QuadTracer<ANY> tr;
-        tr.begin(S, o, d, tmin, tmax, rflags);
-        while (!tr.step(qs)) {
-        }
-        tr.finish();
-        h = tr.h;
-        return h.found;
-    }
-};
-
 // The bounces after the first of every path, in one launch: each lane takes a
 // path from the depth-1 extension queue (ray, slot; throughput, radiance and
 // RNG from the path state) and traces it to its end, then takes the next
@@ -1079,15 +1043,16 @@ struct PathTracer<W, true> {
 // held by its longest path. One loop iteration is one bounce (extension ray,
 // shading, shadow ray). Four waves per SIMD (at most 128 VGPRs): one 1080p
 // frame 3.17 -> 3.03 ms over the unconstrained three.
-template <int W, int BS, bool QUAD>
-__device__ inline void continue_paths(uint32_t* stack, const SceneGPU* __restrict__ scenes, const ViewGPU* __restrict__ views,
+template <int W, int BS>
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_megakernel(const SceneGPU* __restrict__ scenes, const ViewGPU* __restrict__ views,
                                                    uint32_t nv, const float4* __restrict__ q_o, const float4* __restrict__ q_d,
                                                    const uint32_t* __restrict__ q_slot, const uint32_t* __restrict__ count,
                                                    uint32_t* __restrict__ head, uint32_t seg, uint32_t refill,
                                                    const float4* __restrict__ Tin, const uint2* __restrict__ rngs,
                                                    float4* __restrict__ Lout, unsigned long long* __restrict__ stats,
                                                    uint32_t* __restrict__ spill, uint32_t depth0) {
-    const PathTracer<W, QUAD> pt(stack, spill, BS);
+    __shared__ uint32_t stack[kLdsStack * BS];
+    const LaneStack stk = lane_stack<BS>(stack, spill);
     QueueCursor qc(count, head, seg, refill);
     unsigned long long n_ext = 0, n_sh = 0;
     bool active = false;
@@ -1096,7 +1061,7 @@ __device__ inline void continue_paths(uint32_t* stack, const SceneGPU* __restric
     float tmin = 0.001f;
     RNG rng{0u, 0u};
     for (;;) {
-        const uint32_t nq = qc.template next<QUAD>(!active);
+        const uint32_t nq = qc.next(!active);
         if (nq != kNoEntry) {
             slot = q_slot[nq];
             view = nv == 1 ? 0u : find_view(views, nv, slot);
@@ -1119,7 +1084,7 @@ __device__ inline void continue_paths(uint32_t* stack, const SceneGPU* __restric
             bool finish = false;
             HitRec h;
             n_ext++;
-            pt.template trace<false>(S, o, d, tmin, 10000.0f, rflags, h);
+            trace_ray<W, false>(S, o, d, tmin, 10000.0f, rflags, h, stk);
             if (!h.found) {
                 Lp = Lp + T * sample_env(S, d);
                 finish = true;
@@ -1154,16 +1119,15 @@ __device__ inline void continue_paths(uint32_t* stack, const SceneGPU* __restric
                 if (sr.want) {
                     HitRec sh;
                     n_sh++;
-                    if (!pt.template trace<true>(S, sr.o, sr.d, sr.tmin, sr.tmax, sr.flags, sh)) Lp = Lp + sr.contrib;
+                    if (!trace_ray<W, true>(S, sr.o, sr.d, sr.tmin, sr.tmax, sr.flags, sh, stk)) Lp = Lp + sr.contrib;
                 }
             }
             if (finish) {
-                if (!QUAD || (lane_id() & 3u) == 0u) Lout[slot] = make_float4(Lp.x, Lp.y, Lp.z, 0.f);
+                Lout[slot] = make_float4(Lp.x, Lp.y, Lp.z, 0.f);
                 active = false;
             }
         }
     }
-    if (QUAD && (lane_id() & 3u) != 0u) n_ext = n_sh = 0;   // a quad counts its rays once
     for (int off = 32; off > 0; off >>= 1) {
         n_ext += __shfl_xor(n_ext, off);
         n_sh += __shfl_xor(n_sh, off);
@@ -1174,18 +1138,6 @@ __device__ inline void continue_paths(uint32_t* stack, const SceneGPU* __restric
     }
 }
 
-template <int W, int BS>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_megakernel(const SceneGPU* __restrict__ scenes, const ViewGPU* __restrict__ views,
-                                                   uint32_t nv, const float4* __restrict__ q_o, const float4* __restrict__ q_d,
-                                                   const uint32_t* __restrict__ q_slot, const uint32_t* __restrict__ count,
-                                                   uint32_t* __restrict__ head, uint32_t seg, uint32_t refill,
-                                                   const float4* __restrict__ Tin, const uint2* __restrict__ rngs,
-                                                   float4* __restrict__ Lout, unsigned long long* __restrict__ stats,
-                                                   uint32_t* __restrict__ spill, uint32_t depth0) {
-    __shared__ uint32_t stack[kLdsStack * BS];
-    continue_paths<W, BS, false>(stack, scenes, views, nv, q_o, q_d, q_slot, count, head, seg, refill, Tin, rngs, Lout,
-                                             stats, spill, depth0);
-}
 
 // Debug / parity entry points ------------------------------------------------
 template <int W>
