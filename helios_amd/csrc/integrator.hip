@@ -534,11 +534,16 @@ __device__ inline void flush_counts(const TravCount& tc, unsigned long long* out
 // Lanes step their rays independently, so a wave is not held by its longest
 // ray. (Claiming larger private chunks per atomic was measured slower: it
 // starves waves of work when the deep-bounce queues are short.)
-// An exhausted segment costs a wave one failing atomic and the walk over the
-// segments spreads the waves that run dry: reading a head before its atomic
-// (18.4 against 17.8 ms for 20 frames of the 1080p field) and one look at all
-// 32 heads to skip the exhausted ones (18.5 ms: the waves that look together
-// go to the same few segments) were both slower.
+// In passes of up to about 4 M paths (segments of at most kPeekSegment entries)
+// a head is read before its claim: the waves that run dry together would queue
+// up to 8,192 failing atomics on each head, up to 90 us a launch (857 K paths
+// of 6 bounces: 1551 us without the read, 1262 with it; 2.07 M paths of the
+// field 2503 and 2440). Longer passes run dry over a longer time and claim
+// more often, and there the read costs more (20 frames of the 1080p field,
+// 41 M paths: 18.4 ms with it, 17.8 without). One look at all 32 heads to skip
+// the exhausted ones was slower than both (the waves that look together go to
+// the same few segments).
+constexpr uint32_t kPeekSegment = 131072;
 struct QueueCursor {
     const uint32_t* count;  // segment lengths, kCtrStride apart
     uint32_t* head;         // segment read heads, kCtrStride apart
@@ -562,7 +567,11 @@ struct QueueCursor {
             const uint32_t want = nidle - done;
             const uint32_t n = count[shard * kCtrStride];
             uint32_t base = 0;
-            if (idle_lane && rank == 0u) base = atomicAdd(head + shard * kCtrStride, want);
+            if (idle_lane && rank == 0u) {
+                const bool peek = seg <= kPeekSegment;
+                if (peek) base = __hip_atomic_load(head + shard * kCtrStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (!peek || base < n) base = atomicAdd(head + shard * kCtrStride, want);
+            }
             base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)__builtin_ctzll(idle));
             const uint32_t avail = base < n ? min(n - base, want) : 0u;
             if (idle_lane && rank >= done && rank < done + avail) got = shard * seg + base + (rank - done);
@@ -1278,10 +1287,14 @@ __device__ inline float4 output_buffer_value(const SceneGPU& S, uint32_t inst, u
     return make_float4(c.x, c.y, c.z, 1.0f);
 }
 
-// A wave takes 8 x 8 blocks of pixels, whose rays share more of their walks than
-// a row segment's (1920 x 1080 normals of a 249 K triangle scene: 387 -> 352 us;
-// the same blocks as wave-uniform packets took 472 us), and the grid strides
-// over them, so the spill area is a resident grid's.
+// From kViewBlockPixels on a wave takes 8 x 8 blocks of pixels, whose rays share
+// more of their walks than a row segment's (1920 x 1080 normals of a 249 K
+// triangle scene: 387 -> 352 us; 1060 x 870 243 -> 214; 913 x 875 equal; the
+// same blocks as wave-uniform packets took 472 us). Smaller views take 64
+// consecutive pixels: a few waves whose rays are all long hold the launch
+// (633 x 171: 130 us, in blocks 145; 1615 x 335: 178 and 190; but 469 x 533 132
+// and 124). The grid strides over either, so the spill area is a resident grid's.
+constexpr uint32_t kViewBlockPixels = 786432;
 template <int W>
 __global__ void __launch_bounds__(256) k_output_buffer(const SceneGPU* __restrict__ scene, const ViewGPU* __restrict__ view,
                                                        uint32_t w, uint32_t h_, float near_d, float far_d, uint32_t which,
@@ -1290,9 +1303,17 @@ __global__ void __launch_bounds__(256) k_output_buffer(const SceneGPU* __restric
     const LaneStack stk{to_lds(&stack[threadIdx.x]), 256, to_global(spill + blockIdx.x * 256 + threadIdx.x), gridDim.x * 256};
     const ViewGPU& V = *view;
     const SceneGPU& S = *scene;
-    const uint32_t tw = (w + 7u) >> 3, tiles = tw * ((h_ + 7u) >> 3), l = threadIdx.x & 63u;
+    const bool rows = w * h_ < kViewBlockPixels;
+    const uint32_t tw = (w + 7u) >> 3, tiles = rows ? (w * h_ + 63u) >> 6 : tw * ((h_ + 7u) >> 3), l = threadIdx.x & 63u;
     for (uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6); tile < tiles; tile += gridDim.x * 4u) {
-        const uint32_t x = (tile % tw) * 8u + (l & 7u), y = (tile / tw) * 8u + (l >> 3);
+        uint32_t x, y;
+        if (rows) {
+            y = (tile * 64u + l) / w;
+            x = tile * 64u + l - y * w;
+        } else {
+            x = (tile % tw) * 8u + (l & 7u);
+            y = (tile / tw) * 8u + (l >> 3);
+        }
         if (x >= w || y >= h_) continue;
         const float nx = (((float)x + 0.5f) / (float)w) * 2.0f - 1.0f;
         const float ny = (((float)y + 0.5f) / (float)h_) * 2.0f - 1.0f;
@@ -1723,7 +1744,7 @@ hipError_t launch_primary_hits(const LaunchCfg& cfg, const SceneGPU* d_scene, co
     return hipGetLastError();
 }
 
-// Four 8 x 8 pixel blocks per workgroup, at most 16 workgroups per CU (6, 8, 16, 32 per CU: 445, 357, 352, 354 us).
+// Four times 64 pixels (8 x 8 blocks: the more) per workgroup, at most 16 workgroups per CU (6, 8, 16, 32 per CU: 445, 357, 352, 354 us).
 uint32_t output_buffer_blocks(int num_cu, uint32_t w, uint32_t h) {
     return std::min(cdiv(cdiv(w, 8) * cdiv(h, 8), 4), (uint32_t)num_cu * 16u);
 }
