@@ -15,7 +15,7 @@
 //   A (16 x 32)  weights  [Cout][Kpad], k = tap * Cin + c  (lane: row l%16,
 //                k = 8 (l/16) .. +7)
 //   B (32 x 16)  inputs   pixel (l%16) of the tile, channels of k's tap
-//   D (16 x 16)  lane holds pixel l%16, output channels 4 (l/16) .. +3
+//   D (16 x 16)  lane holds pixel l%16, rows 4 (l/16) .. +3 of A
 // The decoder's "upsample, then concatenate with the skip tensor" is not
 // materialized: the B loader reads channels [0, C0) from the low-resolution
 // tensor at (y/2, x/2) and [C0, C0+C1) from the skip tensor.

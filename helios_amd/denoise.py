@@ -42,8 +42,9 @@ def forward_bytes(h, w):
     """Algorithmic HBM bytes of one hh_denoise pass on an h x w surface (padded
     to multiples of 8): every stored tensor read once and written once --
     the packing (radiance + two feature planes in, 16 BF16 channels + the
-    FP32 residual out), the 14 convolutions, the three 2x2 poolings and the
-    head (32 channels + residual in, network output + surface out)."""
+    FP32 residual out), the 14 convolutions, the three 2x2 averages that the
+    convolutions before them also write, and the head on the last one's sums,
+    which are not stored (residual in, surface out)."""
     hp, wp = (h + 7) // 8 * 8, (w + 7) // 8 * 8
 
     def px(lv):
@@ -52,8 +53,8 @@ def forward_bytes(h, w):
     total = px(0) * (48 + 32 + 16)                                       # pack
     for ins, (co, lo) in _CONV_IO:
         total += sum(2 * c * px(lv) for c, lv in ins) + 2 * co * px(lo)
-    total += sum(2 * c * px(lv) + 2 * c * px(lv + 1) for c, lv in _POOLS)
-    total += px(0) * (2 * 32 + 16 + 16 + 16)                            # head
+    total += sum(2 * c * px(lv + 1) for c, lv in _POOLS)
+    total += px(0) * (16 + 16 - 2 * 32)                                 # head instead of the last output
     return total
 
 

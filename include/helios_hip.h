@@ -266,7 +266,8 @@ hh_status hh_scene_add_light(hh_scene scene, const hh_light_desc* desc, uint32_t
 hh_status hh_scene_set_ibl(hh_scene scene, uint32_t size, const float* rgba32f_faces);
 hh_status hh_scene_set_sky(hh_scene scene, const hh_sky_params* params);
 /* Packs the GPU records, builds BLAS per mesh + TLAS on the GPU and bakes the
- * sky. Any later edit marks the scene HIERARCHY_UPDATED and needs a commit. */
+ * sky. Any later edit marks the scene HIERARCHY_UPDATED and needs a commit,
+ * which rebuilds what the edits since the last one touch. */
 hh_status hh_scene_commit(hh_scene scene);
 hh_status hh_scene_num_lights(hh_scene scene, uint32_t* out);
 /* Copies the packed light records (64 B each, scene.cpp:36-42) to host. */
