@@ -1,6 +1,6 @@
 """GPU: traversal with four lanes per ray gives the per-lane traversal's results.
 
-Ray queries of up to 131,072 rays and queue launches with at most 16 rays per
+Ray queries of up to 131,072 rays and queue launches with at most 32 rays per
 wave take four lanes per ray; larger ones, and the counting variant, one. The
 hit is the smallest (t, instance, geometry, primitive) either way, so every
 comparison is exact.
@@ -50,6 +50,26 @@ def test_frames(gpu_ctx, scene, w, h, frames):
         it.render(scene, scene.desc.camera, surf, frames=frames)
         images.append((surf.read(), it.ray_stats()))
     gpu_ctx.set_profiling()
+    assert images[0][0].tobytes() == images[1][0].tobytes()
+    assert images[0][1] == images[1][1]
+    it.close()
+    surf.close()
+
+
+def test_passes_on_both_sides_of_the_head_read(gpu_ctx, scene):
+    """A pass of up to about 4 M paths reads a queue head before it claims, a
+    longer one does not; the image and the ray counts are the same."""
+    from helios_amd import runtime
+    surf = runtime.Surface(gpu_ctx, 1920, 1080)
+    it = runtime.PathIntegrator(gpu_ctx)
+    it.set_max_ray_bounces(3)
+    images = []
+    for in_flight in (1, 3):                 # 2.07 and 6.2 M paths per pass
+        gpu_ctx.set_tuning(frames_in_flight=in_flight)
+        it.restart_bake()
+        it.render(scene, scene.desc.camera, surf, frames=3)
+        images.append((surf.read(), it.ray_stats()))
+    gpu_ctx.set_tuning()
     assert images[0][0].tobytes() == images[1][0].tobytes()
     assert images[0][1] == images[1][1]
     it.close()

@@ -47,6 +47,24 @@ def test_output_buffers_match_oracle(gpu_ctx, oracle_mod, name, desc):
     scene.close()
 
 
+@pytest.mark.parametrize("w,h", [(1023, 768), (1024, 768), (1031, 769)])
+def test_output_buffer_wave_shapes(gpu_ctx, oracle_mod, w, h):
+    """Views of at least 786,432 pixels are traced in 8 x 8 blocks per wave,
+    smaller ones in 64 consecutive pixels: the sizes around the line and a
+    ragged one, with the bar of the views above."""
+    from helios_amd import runtime
+    desc = scenegen.cornell_box(width=w, height=h)
+    scene = runtime.Scene(gpu_ctx, desc)
+    surf = runtime.Surface(gpu_ctx, w, h)
+    runtime.render_output_buffer(scene, desc.camera, OUTPUT_BUFFER_NORMALS, surf)
+    got = surf.read()
+    ref = oracle_mod.OracleScene(desc).output_buffer(OUTPUT_BUFFER_NORMALS)
+    bad = ~np.all(np.abs(got - ref) <= 1e-5 + 1e-5 * np.abs(ref), axis=-1)
+    assert bad.mean() <= 1e-3
+    surf.close()
+    scene.close()
+
+
 def test_final_buffer_is_rejected(gpu_ctx):
     from helios_amd import runtime
     d = scenegen.cornell_box(width=16, height=16)
