@@ -947,6 +947,9 @@ static hh_status build_geometry(hh_scene s, const std::vector<uint32_t>& global_
     HH_HIP(upload(s, geo.allocs, ibase, &geo.ibase));
     HH_HIP(upload(s, geo.allocs, tdesc, &geo.tex));
     HH_HIP(upload(s, geo.allocs, texels, &geo.texels));
+    // optional 64-B quantized BVH4 nodes (same topology and indices): the
+    // BLASes' here, since a later commit may keep them, the TLAS's in every commit
+    if (geo.qnodes) HH_HIP(quantize_bvh4(ctx->stream, d_nodes, geo.qnodes, node_base));
     HH_HIP(hipStreamSynchronize(ctx->stream));
     geo.num_nodes = node_base;
     geo.num_tris = tri_base;
@@ -967,7 +970,6 @@ hh_status hh_scene_commit(hh_scene s) {
     // not reused under another BVH tuning
     if (s->geom.width != W || s->geom.builder != ctx->tune.bvh_builder || s->geom.compressed != ctx->tune.bvh_compressed)
         s->geom.built = false;
-    const bool new_geom = !s->geom.built;
     // ---- packing (scene.cpp:915-1311) -------------------------------------
     std::vector<MaterialData> mat_data;
     std::vector<int32_t> tex_slots;
@@ -1118,7 +1120,7 @@ hh_status hh_scene_commit(hh_scene s) {
     auto& geo = s->geom;
     const size_t node_bytes = W == 8 ? sizeof(WideNode<8>) : sizeof(WideNode<4>);
     hh_status st = HH_OK;
-    if (new_geom) st = build_geometry(s, global_meshes, vbase, ibase, mesh_tris, nv, ni, ntri, tex_slots);
+    if (!geo.built) st = build_geometry(s, global_meshes, vbase, ibase, mesh_tris, nv, ni, ntri, tex_slots);
     if (st != HH_OK) return st;
     void* d_nodes = geo.nodes;
     const std::vector<uint32_t>& blas_root = geo.blas_root;
@@ -1195,13 +1197,10 @@ hh_status hh_scene_commit(hh_scene s) {
     }
     s->bvh_stats[2] = tlas_nodes;
     s->bvh_stats[3] = global_meshes.size();
-    // Optional 64-B quantized BVH4 nodes (same topology and indices): all of
-    // them with new geometry, else the TLAS's.
     int layout = W;
-    if (geo.qnodes) {
-        const uint32_t first = new_geom ? 0u : node_base;
-        HH_HIP(quantize_bvh4(ctx->stream, (char*)d_nodes + size_t(first) * node_bytes, (QNode4*)geo.qnodes + first,
-                             node_base + tlas_nodes - first));
+    if (geo.qnodes) {   // the BLASes' nodes were quantized with the geometry
+        HH_HIP(quantize_bvh4(ctx->stream, (char*)d_nodes + size_t(node_base) * node_bytes, (QNode4*)geo.qnodes + node_base,
+                             tlas_nodes));
         d_nodes = geo.qnodes;
         layout = kLayoutQ4;
     }
