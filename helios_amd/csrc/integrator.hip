@@ -1520,7 +1520,12 @@ struct ProfScope {
 
 // Passes of up to this many paths trace the first bounce's shadow rays and the
 // second's extension rays in one launch (k_trace) too; larger ones overlap two
-// launches on two streams there.
+// launches on two streams there. Frames with two launches and with one, at
+// 131 K paths: 335 and 309 us (Cornell box), 725 and 657 (a field of 249 K
+// triangles), 365 and 334 (textured scene); 262 K: 452 and 462, 880 and 840,
+// 422 and 398; 331 K: 550 and 548, 931 and 930, 446 and 459; 409 K with blocks
+// of 64: 614 and 609, 889 and 902, 444 and 456. (BVH4; see `merge` for the
+// other layouts.)
 constexpr uint32_t kMergePaths = 262144;
 template <int W, int BS, int MODE, bool COUNT>
 static hipError_t frame_impl(const LaunchCfg& cfg, const SceneGPU* d_scenes, const ViewGPU* d_views, const ViewGPU* h_views,
@@ -1530,8 +1535,13 @@ static hipError_t frame_impl(const LaunchCfg& cfg, const SceneGPU* d_scenes, con
     unsigned long long* tc = pf ? pf->d_counts : nullptr;
     if (pf) pf->stats = wf.stats;
     const uint32_t grid = frame_grid(total, cfg.num_cu, cfg.tune.blocks_per_cu, BS);
-    // the traversal launches may give each of two queues' rays four lanes
-    const uint32_t tgrid = frame_grid((uint32_t)std::min<uint64_t>(8ull * total, 0xFFFFFFFFull - BS), cfg.num_cu, cfg.tune.blocks_per_cu, BS);
+    // Traversal launches that can give a ray four lanes are sized for two queues
+    // of such rays. The other layouts' waves hold 64 rays: with eight times the
+    // waves each held a few, and a 256 x 256 frame took 514 instead of 436 us
+    // (BVH8), 528 instead of 466 (compressed).
+    constexpr bool kQuads = W == kLayoutB4 && !COUNT;
+    const uint32_t tgrid =
+        kQuads ? frame_grid((uint32_t)std::min<uint64_t>(8ull * total, 0xFFFFFFFFull - BS), cfg.num_cu, cfg.tune.blocks_per_cu, BS) : grid;
     const uint32_t refill = cfg.tune.refill_lanes;
     // A wave of camera rays holds jittered samples of one or two pixels, which
     // traverse the same nodes and finish together: refilling it only when all
@@ -1598,7 +1608,11 @@ static hipError_t frame_impl(const LaunchCfg& cfg, const SceneGPU* d_scenes, con
                                          ctr + ctr_index(d + 1, kCtrExt, 0), wf.s_o, wf.s_d, wf.s_c, wf.s_slot,
                                          ctr + ctr_index(d, kCtrShadow, 0), wf.feat, wf.capacity);
     };
-    const uint32_t merge = total <= kMergePaths ? 0u : 1u;   // first bounce traced by k_trace
+    // First bounce traced by k_trace. Without quads, small passes keep two
+    // launches on two streams (compressed nodes, 640 x 360: 921 us with one, 899
+    // with two; BVH8, 512 x 512: 609 and 571); from 0.5 M paths one launch is
+    // the faster (724 x 724: 857 and 891; BVH8, 3.7 M paths: 3807 and 3956).
+    const uint32_t merge = total <= kMergePaths ? (kQuads ? 0u : max_bounces) : 1u;
     auto shadow = [&](uint32_t d, hipStream_t sst) {
         ProfScope ps(pf, PK_SHADOW, sst);
         if constexpr (!COUNT) {
@@ -1696,8 +1710,11 @@ hipError_t launch_frame(const LaunchCfg& cfg, const SceneGPU* d_scenes, const Sc
 }
 
 // Ray queries of up to this many rays are traced with four lanes per ray: 8 K
-// waves of 16 rays, what the chip holds at once. 32,768 random rays of a
-// 249 K triangle scene: 138 -> 74 us with the packing of the records.
+// waves of 16 rays, what the chip holds at once. Kernel time with one lane and
+// with four, random rays: 32,768 in a field of 249 K triangles 129 and 65 us,
+// 98,304 148 and 105, 131,072 145 and 116; 131,072 in a field of 15 K triangles
+// 80 and 64, in the Cornell box (36 triangles) 39 and 41. At 196,608 the whole
+// call takes the same either way.
 constexpr uint32_t kQuadTraceMax = 131072;
 hipError_t launch_trace_rays(const LaunchCfg& cfg, const SceneGPU* d_scene, const SceneGPU& h_scene, const float4* d_rays,
                              uint32_t n, uint32_t flags, float4* d_hit, uint32_t* d_ids, uint32_t* spill) {

@@ -74,3 +74,32 @@ def test_passes_on_both_sides_of_the_head_read(gpu_ctx, scene):
     assert images[0][1] == images[1][1]
     it.close()
     surf.close()
+
+
+@pytest.mark.parametrize("tuning", [dict(), dict(bvh_width=8), dict(bvh_compressed=True)])
+@pytest.mark.parametrize("w,h", [(64, 3), (512, 512), (513, 512)])
+def test_frames_around_the_merged_launches(gpu_ctx, tuning, w, h):
+    """Passes of up to 262,144 paths and longer ones share launches between
+    bounces differently, and so do node layouts without quads; the counting
+    variant never shares one. The image and the ray counts are the same."""
+    from helios_amd import runtime
+    before = gpu_ctx.tuning()
+    gpu_ctx.set_tuning(**tuning)
+    try:
+        s = runtime.Scene(gpu_ctx, scenegen.icosphere_field(seed=3, n_spheres=6, level=2, n_leaves=60))
+        surf = runtime.Surface(gpu_ctx, w, h)
+        it = runtime.PathIntegrator(gpu_ctx)
+        it.set_max_ray_bounces(4)
+        images = []
+        for counting in (False, True):
+            gpu_ctx.set_profiling(counting=counting)
+            it.restart_bake()
+            it.render(s, s.desc.camera, surf)
+            images.append((surf.read(), it.ray_stats()))
+        gpu_ctx.set_profiling()
+        assert images[0][0].tobytes() == images[1][0].tobytes()
+        assert images[0][1] == images[1][1]
+        for x in (it, surf, s):
+            x.close()
+    finally:
+        gpu_ctx.set_tuning(**before)
