@@ -1287,50 +1287,62 @@ __device__ inline float4 output_buffer_value(const SceneGPU& S, uint32_t inst, u
     return make_float4(c.x, c.y, c.z, 1.0f);
 }
 
-// From kViewBlockPixels on a wave takes 8 x 8 blocks of pixels, whose rays share
-// more of their walks than a row segment's (1920 x 1080 normals of a 249 K
-// triangle scene: 387 -> 352 us; 1060 x 870 243 -> 214; 913 x 875 equal; the
-// same blocks as wave-uniform packets took 472 us). Smaller views take 64
-// consecutive pixels: a few waves whose rays are all long hold the launch
-// (633 x 171: 130 us, in blocks 145; 1615 x 335: 178 and 190; but 469 x 533 132
-// and 124). The grid strides over either, so the spill area is a resident grid's.
-constexpr uint32_t kViewBlockPixels = 786432;
+// Pixel (x, y) of an output-buffer view.
 template <int W>
+__device__ inline float4 view_pixel(const SceneGPU& S, const ViewGPU& V, uint32_t x, uint32_t y, uint32_t w, uint32_t h_,
+                                    float near_d, float far_d, uint32_t which, const LaneStack& stk) {
+    const float nx = (((float)x + 0.5f) / (float)w) * 2.0f - 1.0f;
+    const float ny = (((float)y + 0.5f) / (float)h_) * 2.0f - 1.0f;
+    float tg[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) tg[r] = (V.vpi[0 * 4 + r] * nx + V.vpi[1 * 4 + r] * ny) + V.vpi[3 * 4 + r];
+    const f3 cam = mk(V.cam[0], V.cam[1], V.cam[2]);
+    const f3 d = normalize(mk(tg[0] / tg[3], tg[1] / tg[3], tg[2] / tg[3]) - cam);
+    // the focal plane's normal is -forward
+    const float cosf_ = -(d.x * V.fplane[0] + d.y * V.fplane[1] + d.z * V.fplane[2]);
+    float4 res = make_float4(0.f, 0.f, 0.f, 1.f);  // clear colour (renderer.cpp:282-287)
+    if (cosf_ > 0.0f) {
+        HitRec hr;
+        trace_ray<W, false>(S, cam, d, near_d / cosf_, far_d / cosf_, HH_TRACE_OPAQUE_BIT, hr, stk);
+        if (hr.found) res = output_buffer_value(S, hr.inst, hr.tri, hr.u, hr.v, which);
+    }
+    return res;
+}
+
+// Views below kViewBlockPixels take 64 consecutive pixels per wave, one thread
+// per pixel (78 VGPRs, six waves per SIMD; as a loop over tiles of either shape
+// it ran at five, 2 to 9 % slower). Larger ones take 8 x 8 blocks, whose rays
+// share more of their walks, and the grid strides over them, so the spill area is
+// a resident grid's (wave-uniform packets of the same blocks: 472 us where the
+// per-lane blocks took 352). In small views the few waves whose rays are all long
+// hold the launch; how far up that goes depends on the scene and the shape. Rows
+// and blocks, two cameras on a field of 249 K triangles and on one of 15 K:
+//   633 x 171     139 160  83  95     161 184  91 105 us
+//   960 x 540     198 239 110 125     199 218 124 140
+//   1024 x 768    214 260 116 136     205 253 119 148
+//   1280 x 720    231 275 128 143     212 253 131 147
+//   1800 x 480    206 247 115 133     196 243 120 142
+//   1366 x 768    257 310 132 148     235 280 129 149
+//   1920 x 1080   342 440 173 198     310 388 160 169
+//   3840 x 300    182 209 103 118     190 216 107 122
+constexpr uint32_t kViewBlockPixels = 786432;
+constexpr uint32_t kViewBlocksPerCu = 16;   // 6, 8, 16, 32: 445, 357, 352, 354 us at 1920 x 1080
+template <int W, bool BLOCKS>
 __global__ void __launch_bounds__(256) k_output_buffer(const SceneGPU* __restrict__ scene, const ViewGPU* __restrict__ view,
                                                        uint32_t w, uint32_t h_, float near_d, float far_d, uint32_t which,
                                                        float4* __restrict__ out, uint32_t* __restrict__ spill) {
     __shared__ uint32_t stack[kLdsStack * 256];
-    const LaneStack stk{to_lds(&stack[threadIdx.x]), 256, to_global(spill + blockIdx.x * 256 + threadIdx.x), gridDim.x * 256};
-    const ViewGPU& V = *view;
-    const SceneGPU& S = *scene;
-    const bool rows = w * h_ < kViewBlockPixels;
-    const uint32_t tw = (w + 7u) >> 3, tiles = rows ? (w * h_ + 63u) >> 6 : tw * ((h_ + 7u) >> 3), l = threadIdx.x & 63u;
-    for (uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6); tile < tiles; tile += gridDim.x * 4u) {
-        uint32_t x, y;
-        if (rows) {
-            y = (tile * 64u + l) / w;
-            x = tile * 64u + l - y * w;
-        } else {
-            x = (tile % tw) * 8u + (l & 7u);
-            y = (tile / tw) * 8u + (l >> 3);
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    const LaneStack stk{to_lds(&stack[threadIdx.x]), 256, to_global(spill + i), gridDim.x * 256};
+    if constexpr (BLOCKS) {
+        const uint32_t tw = (w + 7u) >> 3, tiles = tw * ((h_ + 7u) >> 3), l = threadIdx.x & 63u;
+        for (uint32_t tile = i >> 6; tile < tiles; tile += gridDim.x * 4u) {
+            const uint32_t x = (tile % tw) * 8u + (l & 7u), y = (tile / tw) * 8u + (l >> 3);
+            if (x < w && y < h_) out[y * w + x] = view_pixel<W>(*scene, *view, x, y, w, h_, near_d, far_d, which, stk);
         }
-        if (x >= w || y >= h_) continue;
-        const float nx = (((float)x + 0.5f) / (float)w) * 2.0f - 1.0f;
-        const float ny = (((float)y + 0.5f) / (float)h_) * 2.0f - 1.0f;
-        float tg[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) tg[r] = (V.vpi[0 * 4 + r] * nx + V.vpi[1 * 4 + r] * ny) + V.vpi[3 * 4 + r];
-        const f3 cam = mk(V.cam[0], V.cam[1], V.cam[2]);
-        const f3 d = normalize(mk(tg[0] / tg[3], tg[1] / tg[3], tg[2] / tg[3]) - cam);
-        // the focal plane's normal is -forward
-        const float cosf_ = -(d.x * V.fplane[0] + d.y * V.fplane[1] + d.z * V.fplane[2]);
-        float4 res = make_float4(0.f, 0.f, 0.f, 1.f);  // clear colour (renderer.cpp:282-287)
-        if (cosf_ > 0.0f) {
-            HitRec hr;
-            trace_ray<W, false>(S, cam, d, near_d / cosf_, far_d / cosf_, HH_TRACE_OPAQUE_BIT, hr, stk);
-            if (hr.found) res = output_buffer_value(S, hr.inst, hr.tri, hr.u, hr.v, which);
-        }
-        out[y * w + x] = res;
+    } else {
+        if (i >= w * h_) return;
+        out[i] = view_pixel<W>(*scene, *view, i % w, i / w, w, h_, near_d, far_d, which, stk);
     }
 }
 
@@ -1761,18 +1773,26 @@ hipError_t launch_primary_hits(const LaunchCfg& cfg, const SceneGPU* d_scene, co
     return hipGetLastError();
 }
 
-// Four times 64 pixels (8 x 8 blocks: the more) per workgroup, at most 16 workgroups per CU (6, 8, 16, 32 per CU: 445, 357, 352, 354 us).
+static bool view_rows(uint32_t w, uint32_t h) { return w * h < kViewBlockPixels; }
 uint32_t output_buffer_blocks(int num_cu, uint32_t w, uint32_t h) {
-    return std::min(cdiv(cdiv(w, 8) * cdiv(h, 8), 4), (uint32_t)num_cu * 16u);
+    if (view_rows(w, h)) return cdiv(w * h, 256);
+    return std::min(cdiv(cdiv(w, 8) * cdiv(h, 8), 4), (uint32_t)num_cu * kViewBlocksPerCu);
 }
 hipError_t launch_output_buffer(const LaunchCfg& cfg, const SceneGPU* d_scene, const SceneGPU& h_scene, const ViewGPU* d_view,
                                 uint32_t w, uint32_t h, float near_d, float far_d, uint32_t which, float4* out,
                                 uint32_t* spill) {
     const uint32_t blocks = output_buffer_blocks(cfg.num_cu, w, h);
+    const bool rows = view_rows(w, h);
     const int L = h_scene.bvh_width;
-    if (L == kLayoutB8) k_output_buffer<kLayoutB8><<<blocks, 256, 0, cfg.stream>>>(d_scene, d_view, w, h, near_d, far_d, which, out, spill);
-    else if (L == kLayoutQ4) k_output_buffer<kLayoutQ4><<<blocks, 256, 0, cfg.stream>>>(d_scene, d_view, w, h, near_d, far_d, which, out, spill);
-    else k_output_buffer<kLayoutB4><<<blocks, 256, 0, cfg.stream>>>(d_scene, d_view, w, h, near_d, far_d, which, out, spill);
+#define HH_VIEW(LL)                                                                                                             \
+    do {                                                                                                                        \
+        if (rows) k_output_buffer<LL, false><<<blocks, 256, 0, cfg.stream>>>(d_scene, d_view, w, h, near_d, far_d, which, out, spill); \
+        else k_output_buffer<LL, true><<<blocks, 256, 0, cfg.stream>>>(d_scene, d_view, w, h, near_d, far_d, which, out, spill); \
+    } while (0)
+    if (L == kLayoutB8) HH_VIEW(kLayoutB8);
+    else if (L == kLayoutQ4) HH_VIEW(kLayoutQ4);
+    else HH_VIEW(kLayoutB4);
+#undef HH_VIEW
     return hipGetLastError();
 }
 

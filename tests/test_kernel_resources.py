@@ -1,8 +1,8 @@
 """Register and scratch budgets of the hot kernels, read from the built code.
 
 The traversal, shading and continuation kernels are held to a number of waves
-per SIMD by their VGPR budget (k_extend and k_extend_packet 5, k_shadow 6,
-k_shade and k_megakernel 4). A kernel that outgrows its budget spills to
+per SIMD by their VGPR budget (k_extend and k_extend_packet 5, k_shadow and
+row-wise k_output_buffer 6, k_shade and k_megakernel 4). A kernel that outgrows its budget spills to
 scratch, which puts private-memory traffic into the inner loops (a single
 spilled address cost measurable time here). This reads the AMDGPU kernel
 metadata of the gfx950 code object inside helios_amd/_build/integrator.o
@@ -32,6 +32,9 @@ for bs in (64, 128, 256):
     BUDGETS[f"_ZN2hh15k_extend_packetILi4ELi{bs}EE"] = 96
     BUDGETS[f"_ZN2hh7k_shadeILi{bs}EE"] = 128
     BUDGETS[f"_ZN2hh12k_megakernelILi4ELi{bs}EE"] = 128
+# views of 64 consecutive pixels per wave: six waves (BVH4 and compressed nodes)
+BUDGETS["_ZN2hh15k_output_bufferILi4ELb0EE"] = 80
+BUDGETS["_ZN2hh15k_output_bufferILi16ELb0EE"] = 80
 
 
 def _kernel_metadata(tmp_path):
