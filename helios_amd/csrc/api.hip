@@ -2117,8 +2117,9 @@ hh_status hh_trace_rays_noalloc(hh_scene s, const hh_ray* d_rays, uint32_t n, ui
     float4* d_hit = (float4*)((char*)base + kNoAllocSpillBytes);
     uint32_t* d_ids = (uint32_t*)((char*)base + kNoAllocSpillBytes + kNoAllocHitBytes);
     LaunchCfg cfg{ctx->stream, ctx->num_cu, ctx->tune};
-    // The spill area of a k_trace_rays launch is strided by its thread count,
-    // cdiv(n, 256) * 256 <= kNoAllocMaxRays.
+    // Spill columns: one per thread of k_trace_rays, cdiv(n, 256) * 256, or one
+    // per quad of k_trace_rays_quad, cdiv(n, 16) * 16; either is at most
+    // kNoAllocMaxRays.
     HH_HIP(launch_trace_rays(cfg, s->d_gpu, s->gpu, (const float4*)d_rays, n, flags, d_hit, d_ids, spill));
     HH_HIP(launch_pack_hits(ctx->stream, d_hit, d_ids, n, d_hits));
     return HH_OK;

@@ -578,9 +578,10 @@ struct QuadStack {
     uint32_t spill_stride;
 };
 // `stack` is the block's array of kLdsStack words per thread, `spill` the
-// launch's spill area (at most kQuadStack - kQuadLds words per ray).
+// launch's spill area (kQuadStack - kQuadLds words per quad of the launch, which
+// an area of kSpillStack words per lane or per ray holds).
 __device__ inline QuadStack quad_stack(uint32_t* stack, uint32_t* spill, uint32_t threads_per_block, uint32_t blocks) {
-    static_assert(kQuadStack - kQuadLds <= 4 * kSpillStack, "a quad's spill column fits its four lanes' share");
+    static_assert(kQuadStack - kQuadLds <= kSpillStack, "a quad's spill column fits the share of one lane, and of one ray");
     const uint32_t t = threadIdx.x, lane = t & 63u;
     return {to_lds(stack + (t - lane) * kLdsStack + (lane >> 2)),
             to_global(spill + ((blockIdx.x * threads_per_block + t) >> 2)), (threads_per_block * blocks) >> 2};

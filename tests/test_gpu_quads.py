@@ -3,7 +3,8 @@
 Ray queries of up to 131,072 rays and queue launches with at most 32 rays per
 wave take four lanes per ray; larger ones, and the counting variant, one. The
 hit is the smallest (t, instance, geometry, primitive) either way, so every
-comparison is exact.
+comparison is exact, also for walks deep enough to leave the part of a quad's
+stack that LDS holds (96 entries), up to its capacity of 128.
 """
 import numpy as np
 import pytest
@@ -103,3 +104,64 @@ def test_frames_around_the_merged_launches(gpu_ctx, tuning, w, h):
             x.close()
     finally:
         gpu_ctx.set_tuning(**before)
+
+
+def nested(n):
+    """n instances, each 1.2 times smaller than the last, of n triangles, each
+    1.2 times smaller than the last, all around the origin: binned SAH splits off
+    the largest few at a time, so a ray from the origin into +x, which enters
+    every box and the smallest ones first, holds 3 siblings per node on the way
+    down both trees: 99 entries for n = 140, 121 for 180 and 133 for 200 (a
+    transcription of the split and collapse rules). A triangle covers the part of
+    its box between a diagonal and a point near it, so the closest hits lie among
+    many triangles of the smallest instance, whose boxes are entered first, and
+    rays that miss it walk all the others."""
+    d = scenegen.SceneDesc(sky=(3.0, 0.1, 1.15, 16))
+    d.materials.append(scenegen.material())
+    rng = np.random.default_rng(n)
+    k = np.arange(n)
+    scale = 1.2 ** (n / 2 - k)
+    at, off = rng.uniform(0, 1, n), rng.choice([-1.0, 1.0], n) * rng.exponential(0.1, n)
+    point = np.clip(np.stack([3 * at - 1 + off, 3 * at - 1 - off], 1), -1, 2)
+    pos = np.ones((n, 3, 3))
+    pos[:, 0, 1:], pos[:, 1, 1:], pos[:, 2, 1:] = -1.0, 2.0, point
+    pos = (pos * scale[:, None, None]).reshape(-1, 3)
+    flat = np.tile([-1.0, 0.0, 0.0], (3 * n, 1))
+    d.meshes.append(scenegen._mesh_from_parts([(pos, flat, np.zeros((3 * n, 2)), np.arange(3 * n, dtype=np.uint32), 0)], [0]))
+    for s in scale:
+        d.instances.append((*scenegen.trs(scale=s), 0, -1))
+    return d
+
+
+def into_x(n):
+    rng = np.random.default_rng(n)
+    rays = np.zeros(n, abi.RAY_DTYPE)
+    rays["direction"][:, 0] = 1.0
+    y = rng.uniform(-1.1, 2.1, n)
+    rays["direction"][:, 1] = y
+    rays["direction"][:, 2] = y + rng.normal(0, 0.2, n)
+    rays["tmax"] = 1e15
+    return rays
+
+
+@pytest.mark.parametrize("n", [140, 180])
+def test_walks_that_leave_lds(gpu_ctx, n):
+    from helios_amd import runtime
+    scene = runtime.Scene(gpu_ctx, nested(n))
+    rays = into_x(2048)
+    want = scene.trace_rays(np.resize(rays, QUAD_MAX + 1))[:len(rays)]     # one lane per ray
+    hit = want["t"] >= 0
+    assert 0.3 < hit.mean() < 1.0 and len(np.unique(want["primitive"][hit])) > 16
+    got = scene.trace_rays(rays)
+    assert got.tobytes() == want.tobytes()
+    assert scene.traversal_faults() == dict(lane_stack=0, packet_stack=0, trips=0)
+    scene.close()
+
+
+def test_a_full_stack_ends_the_ray(gpu_ctx):
+    """A walk that needs more than 128 entries is ended and counted."""
+    from helios_amd import runtime
+    scene = runtime.Scene(gpu_ctx, nested(220))
+    scene.trace_rays(into_x(256))
+    assert scene.traversal_faults()["lane_stack"] > 0
+    scene.close()

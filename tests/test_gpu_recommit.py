@@ -87,12 +87,26 @@ def test_recommit_equals_fresh(gpu_ctx, tuning, kinds):
         gpu_ctx.set_tuning(**before)
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 64, 512, 513, 1025])
-def test_tlas_sizes(gpu_ctx, n):
-    """TLAS ranges around one workgroup's 512 primitives: hits of n instances
-    from the GPU builder equal those from the host builder."""
+def same_as_the_host_builder(gpu_ctx, d, rays):
     from helios_amd import runtime
-    n = min(n, 1024)
+    before = gpu_ctx.tuning()
+    hits = []
+    for builder in (3, 1):
+        gpu_ctx.set_tuning(bvh_builder=builder)
+        s = runtime.Scene(gpu_ctx, d)
+        hits.append((s.trace_rays(rays), s.bvh_stats()))
+        s.close()
+    gpu_ctx.set_tuning(**before)
+    assert hits[0][0].tobytes() == hits[1][0].tobytes()
+    assert hits[0][1] == hits[1][1]
+    assert np.any(hits[0][0]["t"] >= 0)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 64, 512, 513, 1023, 1024])
+def test_tlas_sizes(gpu_ctx, n):
+    """TLAS ranges around one and two workgroups' 512 primitives, up to the limit
+    of 1,024 instances: hits and node counts of the GPU builder equal the host
+    builder's."""
     d = scenegen.SceneDesc(sky=(3.0, 0.1, 1.15, 16))
     d.materials.append(scenegen.material())
     m = scenegen.displaced_sphere_mesh(1, 3, 0.05)
@@ -101,14 +115,42 @@ def test_tlas_sizes(gpu_ctx, n):
     rng = np.random.default_rng(n)
     for _ in range(n):
         d.instances.append((*scenegen.trs(rng.uniform(-20, 20, 3), None, rng.uniform(0.5, 2.0)), 0, -1))
-    rays = scenegen.random_rays(4096, (-25, -25, -25), (25, 25, 25), seed=n)
-    before = gpu_ctx.tuning()
-    hits = []
-    for builder in (3, 1):
-        gpu_ctx.set_tuning(bvh_builder=builder)
-        s = runtime.Scene(gpu_ctx, d)
-        hits.append(s.trace_rays(rays))
-        s.close()
-    gpu_ctx.set_tuning(**before)
-    assert hits[0].tobytes() == hits[1].tobytes()
-    assert np.any(hits[0]["t"] >= 0)
+    same_as_the_host_builder(gpu_ctx, d, scenegen.random_rays(4096, (-25, -25, -25), (25, 25, 25), seed=n))
+
+
+@pytest.mark.parametrize("n", [1, 2, 511, 512, 513, 1024, 1025, 4097])
+def test_blas_sizes(gpu_ctx, n):
+    """The same for the triangles of one mesh (beside a mesh of one triangle)."""
+    d = scenegen.SceneDesc(sky=(3.0, 0.1, 1.15, 16))
+    d.materials.append(scenegen.material())
+    rng = np.random.default_rng(n)
+    for k in (n, 1):
+        pos = (rng.uniform(-10, 10, (k, 1, 3)) + rng.normal(0, 1, (k, 3, 3))).reshape(-1, 3)
+        up = np.tile([0.0, 1.0, 0.0], (3 * k, 1))
+        d.meshes.append(scenegen._mesh_from_parts([(pos, up, np.zeros((3 * k, 2)), np.arange(3 * k, dtype=np.uint32), 0)], [0]))
+        d.instances.append((*scenegen.trs((0.0, 0.0, 0.0)), len(d.meshes) - 1, -1))
+    same_as_the_host_builder(gpu_ctx, d, scenegen.random_rays(4096, (-12, -12, -12), (12, 12, 12), seed=n))
+
+
+def test_more_shapes_than_sequences_are_kept(gpu_ctx):
+    """A context keeps 64 captured launch sequences; frames of 70 shapes drop
+    them on the way, and the first shape's image is the same after that."""
+    from helios_amd import runtime
+    d = scenegen.icosphere_field(seed=5, n_spheres=3, level=1, n_leaves=10)
+    scene = runtime.Scene(gpu_ctx, d)
+    it = runtime.PathIntegrator(gpu_ctx)
+    it.set_max_ray_bounces(3)
+
+    surfs = {w: runtime.Surface(gpu_ctx, w, 5) for w in range(16, 16 + 71)}   # destroying one drops sequences too
+
+    def image(w):
+        it.restart_bake()
+        it.render(scene, d.camera, surfs[w], frames=2)
+        return surfs[w].read()
+
+    first = image(16)
+    for w in list(surfs)[1:]:
+        image(w)
+    assert image(16).tobytes() == first.tobytes()
+    for x in (it, *surfs.values(), scene):
+        x.close()

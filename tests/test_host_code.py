@@ -34,3 +34,7 @@ def run(program, tmp_path):
 def test_a_commit_after_a_failed_one_is_complete(tmp_path):
     out = run("commit_retry", tmp_path)
     assert int(out.split()[0]) > 100, out   # every call of twelve kinds of commit was made to fail
+
+
+def test_captured_sequences_are_bounded_and_outlive_commits(tmp_path):
+    run("sequences", tmp_path)
