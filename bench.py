@@ -15,8 +15,9 @@ HBM before timing.
 
 Prints one JSON line (rank 0). Extra fields:
   gsample_bounces_per_s  path segments traced (primary + extension rays) / s
-  roofline               extend (closest-hit traversal) kernel: algorithmic
-                         bytes per launch / measured launch time vs HBM peak
+  roofline               extend (closest-hit traversal) kernels of a profiled
+                         pass: algorithmic bytes per launch / measured launch
+                         time vs HBM peak
   cpu_baseline           the FP32 CPU transcription on this host's cores,
                          on a bounded number of whole frames
   time_to_relmse_0.01    wall time for plain progressive accumulation and for
@@ -78,8 +79,8 @@ def parse():
     p.add_argument("--denoise-probe", action="store_true",
                    help="counter-collection driver: 3 frames with feature planes, then 10 denoiser passes")
     p.add_argument("--probe", action="store_true",
-                   help="counter-collection driver: 2 frames of the workload, then a 1 GiB copy kernel "
-                        "(the calibration point for FETCH_SIZE / WRITE_SIZE)")
+                   help="counter-collection driver: one profiled pass of the workload (the launches that the roofline "
+                        "times), then a 1 GiB copy kernel (the calibration point for FETCH_SIZE / WRITE_SIZE)")
     return p.parse_args()
 
 
@@ -143,8 +144,10 @@ def single_frame(it, scene, desc, surf, pixels, calls=20):
 
 def roofline(ctx, it, scene, desc, surf, chunk, node_bytes, a):
     """Roofline of the closest-hit traversal kernels (k_extend_packet at depth
-    0, k_extend after), on one pass of `chunk` frames: the launch shape of the
-    timed run.
+    0, k_extend after), on one pass of `chunk` frames, profiled: extension and
+    shadow rays have launches of their own there, so that each is timed. The
+    timed frames trace the extension rays of depth 2 and later together with the
+    shadow rays of the bounce before (k_trace).
 
     Pass 1 (HIP events on the launch stream) gives the extension launches'
     time and the rays they traced. Pass 2 (the counting traversal variant,
@@ -157,11 +160,11 @@ def roofline(ctx, it, scene, desc, surf, chunk, node_bytes, a):
     acceleration structure (every BLAS/TLAS node, leaf triangle and instance
     record once): what the launch must move from HBM with ideal caching.
     traffic = HBM bytes per launch measured by FETCH_SIZE / WRITE_SIZE at the
-    same shape (profiles/extend_traffic*.json), scaled by the copy-kernel
-    calibration. The per-lane fetch bytes (every lane's node, triangle and
-    instance fetches) are served mostly by L1/L2 and are reported beside it,
-    as is the issue bound the kernel actually runs into
-    (profiles/extend_issue*.json)."""
+    same shape in the same profiled launches (--probe;
+    profiles/extend_traffic*.json), scaled by the copy-kernel calibration. The
+    per-lane fetch bytes (every lane's node, triangle and instance fetches) are
+    served mostly by L1/L2 and are reported beside it, as is the issue bound the
+    kernel actually runs into (profiles/extend_issue*.json)."""
     ctx.set_profiling(timing=True)
     ctx.reset_profile()
     it.render(scene, desc.camera, surf, frames=chunk)
@@ -203,6 +206,8 @@ def roofline(ctx, it, scene, desc, surf, chunk, node_bytes, a):
         "frac": round(achieved / HBM_PEAK_GBPS, 5), "traffic": traffic,
         "kernel": "k_extend_packet (depth 0) + k_extend (depths 1-%d): closest-hit traversal" % (
             (a.continuation_depth or a.bounces) - 1),
+        "launches": "profiled pass: a launch per kind of ray; the timed frames trace extension depths >= 2 and the "
+                    "shadow rays of the bounce before in one launch (k_trace)",
         "launches_per_pass": ext["launches"], "avg_launch_ms": round(avg_ms, 4),
         "rays_per_launch": round(rays_per_launch),
         "alg_bytes_per_launch": round(alg),
@@ -548,7 +553,9 @@ def main():
         return 0
 
     if a.probe:
+        ctx.set_profiling(timing=True)      # the roofline's launches
         it.render(scene, desc.camera, surf, frames=a.frames_in_flight)
+        ctx.set_profiling()
         ctx.sync()
         gbps = ctx.bandwidth_probe(1 << 30, 1)
         print(json.dumps({"probe": f"{a.frames_in_flight} frames (one chunk) + 1 GiB copy", "copy_gbps": gbps,

@@ -24,7 +24,8 @@ PROBE_BYTES = 1 << 30
 
 def demangle(name):
     """Readable form of the denoiser's mangled template kernel names
-    (_ZN2hh2dn9k_conv3x3ILi48ELi2ELi32ELi32ELi0EE... -> hh::dn::k_conv3x3<48, 2, 32, 32, 0>)."""
+    (_ZN2hh2dn9k_conv3x3ILi48ELi2ELi32ELi32ELi0ENS0_9ConvLargeEEEv... ->
+    hh::dn::k_conv3x3<48, 2, 32, 32, 0, ConvLarge>)."""
     import re
     m = re.match(r"_ZN2hh2dn(\d+)", name)
     if not m:
@@ -32,14 +33,17 @@ def demangle(name):
     n = int(m.group(1))
     rest = name[m.end():]
     kname, tail = rest[:n], rest[n:]
-    args = re.match(r"I((?:Li-?\d+E)+)E", tail)
+    args = re.match(r"I((?:Li-?\d+E)+)(?:NS0_(\d+))?", tail)
     if not args:
         return "hh::dn::" + kname
-    return f"hh::dn::{kname}<{', '.join(re.findall(r'Li(-?[0-9]+)E', args.group(1)))}>"
+    values = re.findall(r"Li(-?[0-9]+)E", args.group(1))
+    if args.group(2):
+        values.append(tail[args.end():args.end() + int(args.group(2))])
+    return f"hh::dn::{kname}<{', '.join(values)}>"
 
 
 def short(name):
-    name = demangle(name)
+    name = demangle(name).replace("(anonymous namespace)::", "")
     n = name.split("(")[0].replace("void ", "")
     return n if len(n) < 90 else n[:87] + "..."
 
@@ -56,25 +60,38 @@ def stats_md(csv_path, cmd, top=12):
 
 
 def passes_md(trace_csv, max_rows=12):
-    """Extension launches (k_extend_packet + k_extend, not the counting
-    instantiations) grouped by wavefront pass: a pass starts at each
-    k_generate dispatch. Lists launches and average duration per pass, in
-    dispatch order, so the timed pass can be matched with the bench's
-    HIP-event figure."""
+    """Traversal launches (not the counting instantiations) grouped by wavefront
+    pass: a pass starts at each k_generate dispatch. Extension launches are
+    k_extend_packet and k_extend; a shared launch (k_trace) traces the shadow rays
+    of one bounce and the extension rays of the next, or, in frames profiled with
+    events, shadow rays alone. Lists launches and average duration per pass, in
+    dispatch order, so the profiled pass can be matched with the bench's HIP-event
+    figure."""
     rows = sorted(csv.DictReader(open(trace_csv)), key=lambda r: int(r["Start_Timestamp"]))
     passes, cur = [], None
     for r in rows:
         n = r["Kernel_Name"]
+        us = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
         if "k_generate<" in n:
-            cur = {"gen": short(n), "ext": []}
+            cur = {"gen": short(n), "ext": [], "shared": [], "shadow": []}
             passes.append(cur)
-        elif cur is not None and ("k_extend_packet<" in n or ("k_extend<" in n and "false>" in n)):
-            cur["ext"].append(int(r["End_Timestamp"]) - int(r["Start_Timestamp"]))
-    lines = ["", "Extension launches per wavefront pass (a pass starts at each k_generate dispatch):", "",
-             "| pass | generate | extension launches | avg us |", "|---|---|---|---|"]
+        elif cur is None or "true>" in n:
+            continue
+        elif "k_extend_packet<" in n or "k_extend<" in n:
+            cur["ext"].append(us)
+        elif "k_trace<" in n:
+            cur["shared"].append(us)
+        elif "k_shadow<" in n:
+            cur["shadow"].append(us)
+
+    def cells(v):
+        return f"{len(v)} | {sum(v) / len(v):.1f}" if v else "0 | -"
+
+    lines = ["", "Traversal launches per wavefront pass (a pass starts at each k_generate dispatch); average us of each kind:",
+             "", "| pass | generate | extension | us | shared (k_trace) | us | shadow | us |", "|---|---|---|---|---|---|---|---|"]
     for i, pz in enumerate(passes[:max_rows]):
         if pz["ext"]:
-            lines.append(f"| {i + 1} | {pz['gen']} | {len(pz['ext'])} | {sum(pz['ext']) / len(pz['ext']) / 1e3:.1f} |")
+            lines.append(f"| {i + 1} | {pz['gen']} | {cells(pz['ext'])} | {cells(pz['shared'])} | {cells(pz['shadow'])} |")
     return "\n".join(lines) + "\n"
 
 
@@ -82,7 +99,7 @@ def timeline_md(trace_csv, pass_no):
     """Every dispatch of wavefront pass `pass_no` (1-based, a pass starts at
     each k_generate dispatch) with its hardware queue, start and end relative
     to the pass's first dispatch, and duration: shows which launches ran side
-    by side (the shadow launch beside the next extension launch)."""
+    by side (the first bounce's shadow launch beside the next extension launch)."""
     rows = sorted(csv.DictReader(open(trace_csv)), key=lambda r: int(r["Start_Timestamp"]))
     starts = [i for i, r in enumerate(rows) if "k_generate<" in r["Kernel_Name"]]
     if pass_no < 1 or pass_no > len(starts):
@@ -211,12 +228,13 @@ def issue(pmc_csv, cmd, simds=1024, xcds=8, cycles_per_valu=4):
       lane_utilization = SQ_THREAD_CYCLES_VALU / (64 x SQ_ACTIVE_INST_VALU):
                          active lanes per issued VALU instruction
       valu_insts_per_wave = SQ_INSTS_VALU / SQ_WAVES
-    GRBM_GUI_ACTIVE is summed over the XCDs."""
+    GRBM_GUI_ACTIVE is summed over the XCDs. k_trace: launches of both kinds of
+    rays, or, in frames profiled with events, of shadow rays alone."""
     agg = per_dispatch_multi(pmc_csv)
     out = {}
     for name, c in agg.items():
         base = name.split("<")[0].split("::")[-1]
-        if base not in ("k_extend", "k_extend_packet", "k_shadow", "k_shade", "k_megakernel") or "true" in name:
+        if base not in ("k_extend", "k_extend_packet", "k_shadow", "k_trace", "k_shade", "k_megakernel") or "true" in name:
             continue
         if any(k not in c for k in ISSUE_COUNTERS):
             continue
