@@ -616,7 +616,10 @@ hh_status hh_denoiser_get_grads(hh_denoiser dn, float* grads, uint64_t n);
  * `out` (same size, RGBA32F, alpha 1). */
 hh_status hh_denoise(hh_denoiser dn, hh_surface in, uint32_t num_frames, hh_surface out);
 /* Host-array entry points: raw records (n x h x w x 12) in, the network
- * output in log(1 + radiance) space (n x h x w x 3) out. */
+ * output in log(1 + radiance) space (n x h x w x 3) out. Like hh_denoise it adds
+ * the last decoder layer's and the head's FP32 sums in another order than a
+ * training step, so the output equals the one a loss was computed from to BF16
+ * rounding, not bit for bit. */
 hh_status hh_denoiser_forward(hh_denoiser dn, const float* feats, uint32_t n, uint32_t h, uint32_t w, float* out_log);
 /* Training loss, mean over pixels and channels (target: n x h x w x 3):
  *   HH_DENOISER_LOSS_LOG_MSE (default)  (out - log(1 + target))^2
